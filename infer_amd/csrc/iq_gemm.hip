@@ -65,7 +65,28 @@ __device__ __forceinline__ uint32_t bf16_pair_int(int a, int b) {
 // BM: activation rows per tile, 128, or 64 for short T (each wave 32 rows).
 // BM = 256 (bf16 activations): 8 waves (4 x 2), each dequantised weight
 // tile in LDS then feeds twice the MFMAs of a 128-row tile.
-template <int KIND, bool XF32, bool FASTW, bool FASTX, int NJ, int BM>
+// MODE: how the operands are loaded.  kAligned: whole 128-column groups and
+// 16-byte aligned rows.  kUnaligned: any K and alignment, the same 16-byte
+// buffer loads at byte offsets (x past the row's end masked to zero, so
+// whatever follows a weight row multiplies zero; the chunk that holds the
+// matrix's last bytes is loaded from the end backwards and shifted); with
+// the K ranges of pick_splits, fp32 activations, int4 1535 x 2050 at T = 70
+// 142 -> 15.6 us, int8 9000 x 9000 at T = 200 1008 -> 280 us against the
+// element-by-element loads on unsplit K that all of these calls took.
+// kBytes: element by element, for rows of under 16 bytes.
+enum { kBytes, kUnaligned, kAligned };
+
+// The 16 bytes v, `n` bytes further on (zeros past the end).
+__device__ __forceinline__ uint4 shift_bytes(uint4 v, uint32_t n) {
+    const uint32_t b = n & 3;
+    uint32_t w0 = __builtin_amdgcn_alignbyte(v.y, v.x, b), w1 = __builtin_amdgcn_alignbyte(v.z, v.y, b);
+    uint32_t w2 = __builtin_amdgcn_alignbyte(v.w, v.z, b), w3 = __builtin_amdgcn_alignbyte(0, v.w, b);
+    if (n & 4) { w0 = w1; w1 = w2; w2 = w3; w3 = 0; }
+    if (n & 8) { w0 = w2; w1 = w3; w2 = 0; w3 = 0; }
+    return n >= 16 ? make_uint4(0, 0, 0, 0) : make_uint4(w0, w1, w2, w3);
+}
+
+template <int KIND, bool XF32, int MODE, int NJ, int BM>
 __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 : 2) void gemm_kernel(const GemmParams p) {
     constexpr int BN = 64 * NJ;
     constexpr int NT = BM == 256 ? 2 * kThreads : kThreads;  // threads
@@ -111,7 +132,7 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
     Regs r0, r1;
 
     // Per-thread source rows, fixed for the whole K loop (a step adds its
-    // column offset): the fast paths need no per-step bounds arithmetic.
+    // column offset): used by kBytes only.
     const uint8_t* wrow[WCH];
     const uint8_t* zrow[WCH];
     bool wok[WCH];
@@ -139,7 +160,7 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
                        : static_cast<const void*>(p.xb + (xok[i] ? m : 0) * p.K + kbeg);
         xcol[i] = XF32 ? (c & 15) * 4 : (c & 7) * 8;  // element offset inside the step
     }
-    // Fast paths: buffer resources over this tile's rows (wave-uniform), so
+    // Otherwise: buffer resources over this tile's rows (wave-uniform), so
     // every global load of the K loop is unconditional (rows past T or N and
     // groups past the range read zero without a memory access).  A load
     // under a branch makes the compiler wait for all outstanding loads
@@ -148,9 +169,15 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
     constexpr int XE = XF32 ? 4 : 2;
     const int64_t xrows = p.T - m0 < BM ? p.T - m0 : BM;
     const int64_t nrows = p.N - n0 < BN ? p.N - n0 : BN;
+    // kUnaligned: a row's last chunk runs into the next row's bytes, up to
+    // the end of the whole matrix
+    const int64_t over = MODE == kUnaligned ? 16 : 0;
+    const int64_t xbytes = std::min(xrows * p.K * XE + over, (p.T - m0) * p.K * XE);
+    const int64_t wbytes = std::min(nrows * row_bytes + over, (p.N - n0) * row_bytes);
+    const bool wlast = MODE == kUnaligned && n0 + BN >= p.N, xlast = MODE == kUnaligned && m0 + BM >= p.T;
     const rsrc_t rx = make_rsrc(XF32 ? static_cast<const void*>(p.xf + m0 * p.K)
-                                     : static_cast<const void*>(p.xb + m0 * p.K), xrows * p.K * XE);
-    const rsrc_t rw = make_rsrc(p.q + n0 * row_bytes, nrows * row_bytes);
+                                     : static_cast<const void*>(p.xb + m0 * p.K), xbytes);
+    const rsrc_t rw = make_rsrc(p.q + n0 * row_bytes, wbytes);
     const rsrc_t rsc = make_rsrc(p.scales + n0 * p.G, nrows * p.G * 2);
     const rsrc_t rzp = make_rsrc(KIND == 1 ? p.zeros + n0 * p.G : nullptr, KIND == 1 ? nrows * p.G : 0);
     uint32_t xoff[XCH], woff[WCH], zoff[WCH];
@@ -159,6 +186,7 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
         const int c = tid + NT * i;
         const int row = XF32 ? c >> 4 : c >> 3;
         xoff[i] = uint32_t((int64_t(row) * p.K + kbeg + xcol[i]) * XE);
+        if (MODE == kUnaligned && !xok[i]) xoff[i] = kOob;
     }
 #pragma unroll
     for (int i = 0; i < WCH; i++) {
@@ -168,6 +196,13 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
         zoff[i] = (KIND == 1 && wok[i]) ? uint32_t(row * p.G + gbeg) : kOob;
     }
 
+    // kUnaligned: the offset a chunk is loaded from, and how far past it the
+    // chunk begins (non-zero only for the chunk over the end of the matrix).
+    // (fp32 x needs neither: its elements are whole dwords, which the buffer
+    // resource cuts off exactly)
+    auto woff_at = [&](int i, uint32_t k0) { return woff[i] + (KIND == 1 ? k0 / 2 : k0); };
+    auto xoff_at = [&](int i, uint32_t k0) { return xoff[i] + k0 * XE; };
+    auto clamp16 = [&](uint32_t off, int64_t bytes) { return off < kOob ? std::min(off, uint32_t(bytes - 16)) : off; };
     auto load_step = [&](Regs& rg, int kt) {
         uint4* xr = rg.xr;
         uint4* wr = rg.wr;
@@ -176,8 +211,10 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
 #pragma unroll
         for (int i = 0; i < XCH; i++) {
             const int64_t k = k0 + xcol[i];
-            if (FASTX) {
-                xr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[i] + uint32_t(k0 * XE), 0, 0));
+            if (MODE != kBytes) {
+                const uint32_t off = xoff_at(i, uint32_t(k0));
+                xr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      rx, MODE == kUnaligned && !XF32 ? clamp16(off, xbytes) : off, 0, 0));
             } else if (XF32) {
                 const float* xp = static_cast<const float*>(xrow[i]);
                 float f[4];
@@ -196,9 +233,10 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
 #pragma unroll
         for (int i = 0; i < WCH; i++) {
             const int64_t off = (KIND == 1 ? k0 / 2 : k0) + wcol[i];
-            if (FASTW) {
+            if (MODE != kBytes) {
+                const uint32_t o16 = woff_at(i, uint32_t(k0));
                 wr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                      rw, woff[i] + uint32_t(KIND == 1 ? k0 / 2 : k0), 0, 0));
+                                                      rw, MODE == kUnaligned ? clamp16(o16, wbytes) : o16, 0, 0));
             } else if (!wok[i]) {
                 wr[i] = make_uint4(0, 0, 0, 0);
             } else {
@@ -211,15 +249,45 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
         }
 #pragma unroll
         for (int i = 0; i < WCH; i++) {
-            if (KIND == 1 && FASTW) zr[i] = __builtin_amdgcn_raw_buffer_load_b8(rzp, zoff[i] + uint32_t(k0 / kGroup), 0, 0);
+            if (KIND == 1 && MODE != kBytes) zr[i] = __builtin_amdgcn_raw_buffer_load_b8(rzp, zoff[i] + uint32_t(k0 / kGroup), 0, 0);
             else zr[i] = (KIND == 1 && wok[i]) ? zrow[i][k0 / kGroup] : 0u;
         }
     };
 
-    auto store_step = [&](const Regs& rg, int buf) {
-        const uint4* xr = rg.xr;
-        const uint4* wr = rg.wr;
+    auto store_step = [&](Regs& rg, int kt, int buf) {
+        uint4* xr = rg.xr;
+        uint4* wr = rg.wr;
         const uint32_t* zr = rg.zr;
+        if (MODE == kUnaligned) {
+            const uint32_t k0 = uint32_t(kt) * BK;
+            if (!XF32 && xlast) {
+#pragma unroll
+                for (int i = 0; i < XCH; i++) {
+                    const uint32_t off = xoff_at(i, k0);
+                    xr[i] = shift_bytes(xr[i], off - clamp16(off, xbytes));
+                }
+            }
+            if (wlast) {
+#pragma unroll
+                for (int i = 0; i < WCH; i++) {
+                    const uint32_t off = woff_at(i, k0);
+                    wr[i] = shift_bytes(wr[i], off - clamp16(off, wbytes));
+                }
+            }
+            if (int64_t(k0) + BK > klen) {  // the row ends inside this step
+#pragma unroll
+                for (int i = 0; i < XCH; i++) {
+                    const int left = int(klen - k0) - xcol[i];  // elements of the row in this chunk
+                    uint32_t d[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        if (XF32) d[e] = e < left ? d[e] : 0u;
+                        else d[e] = 2 * e + 1 < left ? d[e] : (2 * e < left ? d[e] & 0xFFFFu : 0u);
+                    }
+                    xr[i] = make_uint4(d[0], d[1], d[2], d[3]);
+                }
+            }
+        }
 #pragma unroll
         for (int i = 0; i < XCH; i++) {
             const int c = tid + NT * i;
@@ -335,7 +403,7 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
     // after the MFMAs) and those of the other set step kt + 2 (requested one
     // step earlier), so global loads have two steps to arrive.
     load_step(r0, 0);
-    store_step(r0, 0);
+    store_step(r0, 0, 0);
     if (nk > 1) load_step(r1, 1);
     if (nk > 2) load_step(r0, 2);
     __syncthreads();
@@ -384,7 +452,7 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
             }
             load_scales(kt / 2 + 2, s_nxt);
         }
-        if (kt + 1 < nk) store_step(rnext, buf ^ 1);
+        if (kt + 1 < nk) store_step(rnext, kt + 1, buf ^ 1);
         if (kt + 3 < nk) load_step(rnext, kt + 3);
         __syncthreads();
         (void)rlater;
@@ -841,26 +909,25 @@ __global__ __launch_bounds__(256) void gemm_reduce4_kernel(const float* __restri
 }
 
 template <int KIND, bool XF32, int NJ>
-void launch_gemm_t(const GemmParams& p, bool fastw, bool fastx, int bm, hipStream_t stream) {
+void launch_gemm_t(const GemmParams& p, int mode, int bm, hipStream_t stream) {
     const unsigned grid = unsigned(p.tiles_m * p.tiles_n * p.splits);
     if constexpr (!XF32) {
-        if (bm == 256) {  // (fast paths only)
-            gemm_kernel<KIND, XF32, true, true, NJ, 256><<<grid, 2 * kThreads, 0, stream>>>(p);
+        if (bm == 256) {  // (aligned only)
+            gemm_kernel<KIND, XF32, kAligned, NJ, 256><<<grid, 2 * kThreads, 0, stream>>>(p);
             return;
         }
     }
-    if (bm == 64) gemm_kernel<KIND, XF32, true, true, NJ, 64><<<grid, kThreads, 0, stream>>>(p);  // (fast paths only)
-    else if (fastw && fastx) gemm_kernel<KIND, XF32, true, true, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
-    else if (fastw) gemm_kernel<KIND, XF32, true, false, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
-    else if (fastx) gemm_kernel<KIND, XF32, false, true, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
-    else gemm_kernel<KIND, XF32, false, false, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
+    if (mode == kBytes) gemm_kernel<KIND, XF32, kBytes, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
+    else if (mode == kUnaligned && bm == 64) gemm_kernel<KIND, XF32, kUnaligned, NJ, 64><<<grid, kThreads, 0, stream>>>(p);
+    else if (mode == kUnaligned) gemm_kernel<KIND, XF32, kUnaligned, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
+    else if (bm == 64) gemm_kernel<KIND, XF32, kAligned, NJ, 64><<<grid, kThreads, 0, stream>>>(p);
+    else gemm_kernel<KIND, XF32, kAligned, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
 }
 
 // Few output tiles (short T): split K into ranges of whole 128-column groups
 // so that the tiles x ranges fill the workgroup slots of the CUs (per_cu
 // resident workgroups of the instance per CU) in one round, the range sums
-// added by gemm_reduce_kernel; needs the fast (aligned) paths and room for
-// the sums.  Rounding the range count down rather than up keeps a second,
+// added by gemm_reduce_kernel; needs room for the sums.  Rounding the range count down rather than up keeps a second,
 // mostly idle round of workgroups off the critical path (7B down 3584 x
 // 18944 at T = 80 / 200, fp32 activations: 76.8 / 140.6 -> 60.7 / 111.0
 // us; bf16 activations 50.1 / 94.9 -> 36.6 / 69.4 us; 7B gate 18944 x 3584
@@ -889,12 +956,12 @@ int pick_splits(int tiles, int slots, int64_t G, int64_t T, int64_t N, int64_t p
     return S;
 }
 
-void plan_splits(GemmParams& p, bool fast, int64_t part_floats, int per_cu) {
+void plan_splits(GemmParams& p, int64_t part_floats, int per_cu) {
     p.splits = 1;
     p.kchunk = p.K;
     const int tiles = p.tiles_m * p.tiles_n, want = per_cu * device_cu_count();
-    if (!fast || !p.part) return;
-    const int64_t G = p.K / kGroup;
+    if (!p.part) return;
+    const int64_t G = p.G;
     const int S = pick_splits(tiles, want, G, p.T, p.N, part_floats);
     if (S < 2 || G < 2) return;
     const int64_t gch = (G + S - 1) / S;
@@ -903,7 +970,7 @@ void plan_splits(GemmParams& p, bool fast, int64_t part_floats, int per_cu) {
 }
 
 template <int KIND, bool XF32>
-void launch_gemm_nj(GemmParams& p, bool fastw, bool fastx, int bm, int64_t part_floats, hipStream_t stream) {
+void launch_gemm_nj(GemmParams& p, int mode, int bm, int64_t part_floats, hipStream_t stream) {
     // 128-wide tiles unless they leave CUs without two workgroups to run;
     // with 64-row tiles (short T) always, the K split filling the CUs: each
     // workgroup then re-reads the activations for twice the columns (7B int8
@@ -920,12 +987,12 @@ void launch_gemm_nj(GemmParams& p, bool fastw, bool fastx, int bm, int64_t part_
     const bool nj2_rounds = 2 * ((t128 + slots - 1) / slots) <= (t64 + slots - 1) / slots;
     if (t128 >= 2 * device_cu_count() || bm == 64 || nj2_rounds) {
         p.tiles_n = int((p.N + 127) / 128);
-        plan_splits(p, fastw && fastx, part_floats, per_cu);
-        launch_gemm_t<KIND, XF32, 2>(p, fastw, fastx, bm, stream);
+        plan_splits(p, part_floats, per_cu);
+        launch_gemm_t<KIND, XF32, 2>(p, mode, bm, stream);
     } else {
         p.tiles_n = int((p.N + 63) / 64);
-        plan_splits(p, fastw && fastx, part_floats, per_cu);
-        launch_gemm_t<KIND, XF32, 1>(p, fastw, fastx, bm, stream);
+        plan_splits(p, part_floats, per_cu);
+        launch_gemm_t<KIND, XF32, 1>(p, mode, bm, stream);
     }
     if (p.splits > 1) {
         const int64_t n = p.T * p.N;
@@ -1071,9 +1138,12 @@ hipError_t launch_gemm(const float* x_f32, const uint16_t* x_bf16, const QView& 
     p.xf = x_f32; p.xb = x_bf16;
     p.q = W.q; p.scales = W.scales; p.zeros = W.zeros; p.bias = bias; p.y = y;
     p.T = T; p.N = W.rows; p.K = W.cols; p.G = W.groups;
-    const bool fastw = (p.K % kGroup == 0);
     const uintptr_t xa = x_f32 ? reinterpret_cast<uintptr_t>(x_f32) : reinterpret_cast<uintptr_t>(x_bf16);
-    const bool fastx = (p.K % BK == 0) && (xa % 16 == 0);
+    // (kUnaligned: rows of at least one 16-byte chunk, 128 of them within a
+    // buffer resource's 2 GiB)
+    const int64_t least = W.kind == 1 ? 32 : 16;
+    const int mode = p.K % kGroup == 0 && xa % 16 == 0 ? kAligned
+                     : p.K >= least && p.K < (int64_t(1) << 22) ? kUnaligned : kBytes;
     // 64-row tiles for short T (less MFMA work on padding rows, more tiles):
     // 7B int8, fp32 activations, gate 18944 x 3584 at T = 33 / 64 / 128 /
     // 256: 115 / 113 / 137 / 202 -> 55 / 58 / 97 / 139 us; down 3584 x
@@ -1087,15 +1157,15 @@ hipError_t launch_gemm(const float* x_f32, const uint16_t* x_bf16, const QView& 
     // int8 down 269 / 249 us (one 8-wave workgroup per CU leaves the step
     // barriers uncovered, which costs more than the conversion saves on a
     // wide matrix or with int8's cheaper conversion).
-    const bool big = !x_f32 && fastw && fastx && T >= 512 && W.kind == 1 && W.rows < 8192;
-    const int bm = (short_t && fastw && fastx) ? 64 : (big ? 256 : 128);
+    const bool big = !x_f32 && mode == kAligned && T >= 512 && W.kind == 1 && W.rows < 8192;
+    const int bm = (short_t && mode != kBytes) ? 64 : (big ? 256 : 128);
     p.tiles_m = int((T + bm - 1) / bm);
     if (x_f32) {
-        if (W.kind == 1) launch_gemm_nj<1, true>(p, fastw, fastx, bm, ws->part_floats, stream);
-        else launch_gemm_nj<0, true>(p, fastw, fastx, bm, ws->part_floats, stream);
+        if (W.kind == 1) launch_gemm_nj<1, true>(p, mode, bm, ws->part_floats, stream);
+        else launch_gemm_nj<0, true>(p, mode, bm, ws->part_floats, stream);
     } else {
-        if (W.kind == 1) launch_gemm_nj<1, false>(p, fastw, fastx, bm, ws->part_floats, stream);
-        else launch_gemm_nj<0, false>(p, fastw, fastx, bm, ws->part_floats, stream);
+        if (W.kind == 1) launch_gemm_nj<1, false>(p, mode, bm, ws->part_floats, stream);
+        else launch_gemm_nj<0, false>(p, mode, bm, ws->part_floats, stream);
     }
     return hipGetLastError();
 }

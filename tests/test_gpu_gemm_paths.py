@@ -1,0 +1,73 @@
+"""The prefill GEMM's load paths at their edges, against the oracle's
+float64 linear over dequant() with the reference's conditioning tolerance
+(tests/test_ops_gpu.cu:199-206)."""
+import numpy as np
+import pytest
+import torch
+
+from infer_amd import ops
+from oracle import oracle as O
+from tests.gpu_util import QFix, bias_of, check_linear, out_buffer, say
+
+pytestmark = pytest.mark.gpu
+
+
+def shifted(a, by):
+    """The array on the device, starting `by` elements into its allocation
+    and ending with it."""
+    t = torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    buf = torch.zeros(t.numel() + by, dtype=t.dtype, device="cuda")
+    buf[by:] = t.view(-1)
+    return buf[by:]
+
+
+# (N, K): rows of one 16-byte chunk and less, rows that end inside a chunk
+# and inside a dword, one row past a tile, K of one step and a bit, several
+# K ranges; whole groups, for unaligned inputs
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("N,K", [(1, 14), (3, 16), (5, 30), (2, 32), (129, 34), (64, 66), (65, 130), (257, 1022),
+                                 (31, 2050), (128, 256)])
+def test_unaligned_rows(kind, N, K):
+    rng = np.random.default_rng(1000 * N + K + kind)
+    Ks = [K] if kind == 1 or K % 128 == 0 else [K, K + 1]  # int8 rows of odd length too
+    for k in Ks:
+        W = QFix(rng, N, k, kind)
+        bb, bd = bias_of(rng, N)
+        for T in (33, 70, 129):
+            x = rng.standard_normal((T, k), dtype=np.float32)
+            for by in (0, 1):
+                y = out_buffer(T, N)
+                say("unaligned fp32", kind, N, k, T, by)
+                ops.launch_gemm_tiled_q(shifted(x, by), W.view, bd, T, k, N, y)
+                torch.cuda.synchronize()
+                check_linear(y, x, W, bb, T, f"fp32 kind={kind} {N}x{k} T={T} +{by}")
+                xb = O.f32_to_bf16(x)
+                y = out_buffer(T, N)
+                say("unaligned bf16", kind, N, k, T, by)
+                ops.launch_gemm_bf16x(shifted(xb.view(np.int16), by), W.view, bd, T, k, N, y)
+                torch.cuda.synchronize()
+                check_linear(y, O.bf16_to_f32(xb), W, bb, T, f"bf16 kind={kind} {N}x{k} T={T} +{by}")
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_unaligned_rows_ignore_what_follows(kind):
+    """The columns past a row's end are the next row's: non-finite values
+    there (the next activation row) must not reach this row's outputs."""
+    N, K, T = 40, 202, 66
+    rng = np.random.default_rng(9 + kind)
+    W = QFix(rng, N, K, kind)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    x[1::2] = np.inf
+    want, _ = O.linear_dq_f64(x[0::2], W.dq, None)
+    for bf16 in (False, True):
+        xs = O.f32_to_bf16(x) if bf16 else x
+        y = out_buffer(T, N)
+        if bf16:
+            ops.launch_gemm_bf16x(torch.from_numpy(xs.view(np.int16)).cuda(), W.view, None, T, K, N, y)
+            want, _ = O.linear_dq_f64(O.bf16_to_f32(xs)[0::2], W.dq, None)
+        else:
+            ops.launch_gemm_tiled_q(torch.from_numpy(xs).cuda(), W.view, None, T, K, N, y)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()[:T * N].reshape(T, N)
+        assert np.all(np.isfinite(got[0::2])) and not np.any(np.isfinite(got[1::2]))
+        assert np.abs(got[0::2] - want).max() <= 5e-6 * np.abs(want).max() * 8
