@@ -84,6 +84,34 @@ __device__ __forceinline__ void dq_int4_x8(uint32_t v, uint32_t zb, uint32_t zc,
 __device__ __forceinline__ uint32_t zpair_1024(uint32_t z) { return (0xE400u + z) * 0x00010001u; }
 __device__ __forceinline__ uint32_t zpair_64(uint32_t z) { return (0xD400u + 16u * z) * 0x00010001u; }
 
+// int8: 4 codes (one dword) -> 2 dwords of bf16 pairs in column order,
+// exact: the fp32 of an integer below 256 in magnitude is its bf16 and 16
+// zero bits (one conversion per code, one byte permute per two).
+__device__ __forceinline__ void bf16_int8_x4(uint32_t d, uint32_t& lo, uint32_t& hi) {
+    const uint32_t f0 = __float_as_uint(float(int8_t(d))), f1 = __float_as_uint(float(int8_t(d >> 8)));
+    const uint32_t f2 = __float_as_uint(float(int8_t(d >> 16))), f3 = __float_as_uint(float(int8_t(d >> 24)));
+    lo = __builtin_amdgcn_perm(f1, f0, 0x07060302u);
+    hi = __builtin_amdgcn_perm(f3, f2, 0x07060302u);
+}
+
+// int4: 8 nibbles (one dword, columns c..c+7) -> 4 dwords of bf16 pairs of
+// q - z in column order, exact: q - z as signed bytes (128 + q - z has no
+// carry), then as int8.
+__device__ __forceinline__ void bf16_int4_x8(uint32_t v, uint32_t z, uint32_t& o0, uint32_t& o1, uint32_t& o2,
+                                             uint32_t& o3) {
+    const uint32_t zb = (0x80u - z) * 0x01010101u;
+    const uint32_t e = ((v & 0x0F0F0F0Fu) + zb) ^ 0x80808080u;         // columns 0, 2, 4, 6
+    const uint32_t o = (((v >> 4) & 0x0F0F0F0Fu) + zb) ^ 0x80808080u;  // columns 1, 3, 5, 7
+    auto pair = [&](int i) {
+        const uint32_t a = __float_as_uint(float(int8_t(e >> (8 * i)))), b = __float_as_uint(float(int8_t(o >> (8 * i))));
+        return __builtin_amdgcn_perm(b, a, 0x07060302u);
+    };
+    o0 = pair(0);
+    o1 = pair(1);
+    o2 = pair(2);
+    o3 = pair(3);
+}
+
 // Position inside an 8-column octet of the int4 operand order above:
 // operand slot i holds column perm8(i).
 __host__ __device__ constexpr int perm8(int i) { return (i >> 1) + 4 * (i & 1); }

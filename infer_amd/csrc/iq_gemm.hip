@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "iq_gemm.h"
 #include "iq_internal.h"
 #include "iq_limbs.h"
 
@@ -1003,6 +1004,22 @@ void launch_gemm_nj(GemmParams& p, int mode, int bm, int64_t part_floats, hipStr
     }
 }
 
+// Estimated time of tiles x S K ranges on the narrow tiles, workgroups of
+// which per_cu share a CU, group_us a group and round (measured: 7B gate
+// 18944 x 3584, T = 201 and 384..1024), plus the range sums' way through
+// memory: what the wide tiles' estimate is compared with (GemmwPlan).  Both
+// sides at the line, fp32 int8: 7B gate at T = 160 / 201 86 / 120 -> 86
+// (kept) / 105 us, o 3584 x 3584 at T = 384 / 512 47 / 55 -> 46 / 52, 1.5B
+// gate 8960 x 1536 at T = 384 / 512 45 (kept) / 66 -> 44 / 57; bf16: 7B gate
+// at T = 300 / 384 80 / 83 (kept) against 88 / 112 on the wide tiles, at T =
+// 450 133 -> 113.
+double narrow_us(int tiles, int per_cu, int S, int64_t G, int64_t T, int64_t N, double group_us) {
+    const int slots = per_cu * device_cu_count();
+    const int64_t gch = (G + S - 1) / S;
+    return 4.0 + double((int64_t(tiles) * S + slots - 1) / slots) * double(gch) * group_us +
+           (S > 1 ? 5.0 + double(S) * double(T) * double(N) * 8 / 9e6 : 0.0);
+}
+
 // The fp16 operand path (K % 128 == 0, 16-byte aligned activations): one
 // preparation launch, the GEMM, and the range sums when K is split, for T
 // rows whose operands fit the workspace's operand area.
@@ -1063,6 +1080,16 @@ hipError_t launch_gemmh_chunk(const float* x_f32, const QView& W, const uint16_t
                 p.splits = int((G + gch - 1) / gch);
             }
         }
+    }
+    if (T > 64 && reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
+        GemmwParams w;
+        w.a = reinterpret_cast<const uint16_t*>(ah); w.al = reinterpret_cast<const uint16_t*>(al); w.rs = rs;
+        w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
+        w.T = T; w.N = W.rows; w.K = K; w.G = W.groups;
+        if (launch_gemmw(w, W.kind, narrow_us(p.tiles_m * p.tiles_n, bm == 128 ? 1 : 2, p.splits, W.groups, T, p.N,
+                                              bm == 128 ? (W.kind == 1 ? 2.45 : 2.65) : (W.kind == 1 ? 2.05 : 2.4)),
+                         ws->part_floats, stream))
+            return hipGetLastError();
     }
     const unsigned ggrid = unsigned(p.tiles_m * p.tiles_n * p.splits);
     if (bm == 128) {
@@ -1159,6 +1186,16 @@ hipError_t launch_gemm(const float* x_f32, const uint16_t* x_bf16, const QView& 
     // wide matrix or with int8's cheaper conversion).
     const bool big = !x_f32 && mode == kAligned && T >= 512 && W.kind == 1 && W.rows < 8192;
     const int bm = (short_t && mode != kBytes) ? 64 : (big ? 256 : 128);
+    if (!x_f32 && mode == kAligned && T > 64 && reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
+        GemmwParams w;
+        w.a = x_bf16; w.al = nullptr; w.rs = nullptr;
+        w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
+        w.T = T; w.N = W.rows; w.K = p.K; w.G = W.groups;
+        const int rows = bm == 256 ? 128 : bm, tiles = int((T + rows - 1) / rows) * int((p.N + 127) / 128);
+        const int S = pick_splits(tiles, 2 * device_cu_count(), p.G, T, p.N, ws->part_floats);
+        if (launch_gemmw(w, W.kind, narrow_us(tiles, 2, S, p.G, T, p.N, bm == 64 ? 1.9 : 2.8), ws->part_floats, stream))
+            return hipGetLastError();
+    }
     p.tiles_m = int((T + bm - 1) / bm);
     if (x_f32) {
         if (W.kind == 1) launch_gemm_nj<1, true>(p, mode, bm, ws->part_floats, stream);

@@ -71,3 +71,58 @@ def test_unaligned_rows_ignore_what_follows(kind):
         got = y.cpu().numpy()[:T * N].reshape(T, N)
         assert np.all(np.isfinite(got[0::2])) and not np.any(np.isfinite(got[1::2]))
         assert np.abs(got[0::2] - want).max() <= 5e-6 * np.abs(want).max() * 8
+
+
+# The wide tiles (iq_gemmw.hip): 128- and 256-row tiles of bf16 and 128-row
+# tiles of fp32 activations, all K ranges of split tiles, rows and columns
+# past the last tile, N that is no multiple of 4 (the reduction's scalar
+# stores); whole rounds of tiles beside split ones are in test_gpu_routes
+# (the 7B gate at T = 1024).
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("N,K,Ts", [(18947, 3584, (100, 201)), (3587, 18944, (257, 450)), (8192, 4096, (513,))])
+def test_wide_tiles(kind, N, K, Ts):
+    rng = np.random.default_rng(N + kind)
+    W = QFix(rng, N, K, kind, sd=0.02)
+    bb, bd = bias_of(rng, N)
+    for T in Ts:
+        x = rng.standard_normal((T, K), dtype=np.float32)
+        x[:, rng.integers(0, K, 3)] *= 40.0
+        y = out_buffer(T, N)
+        say("wide tiles fp32", kind, N, K, T)
+        ops.launch_gemm_tiled_q(torch.from_numpy(x).cuda(), W.view, bd, T, K, N, y)
+        torch.cuda.synchronize()
+        check_linear(y, x, W, bb, T, f"wide fp32 kind={kind} {N}x{K} T={T}")
+        xb = O.f32_to_bf16(x)
+        y = out_buffer(T, N)
+        say("wide tiles bf16", kind, N, K, T)
+        ops.launch_gemm_bf16x(torch.from_numpy(xb.view(np.int16)).cuda(), W.view, bd, T, K, N, y)
+        torch.cuda.synchronize()
+        check_linear(y, O.bf16_to_f32(xb), W, bb, T, f"wide bf16 kind={kind} {N}x{K} T={T}")
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_wide_tiles_non_finite_rows(kind):
+    """A row with inf or NaN gives a non-finite output row and leaves the
+    other rows as they are."""
+    N, K, T = 8192, 4096, 513
+    rng = np.random.default_rng(77 + kind)
+    W = QFix(rng, N, K, kind, sd=0.02)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    bad = x.copy()
+    bad[5, 100], bad[300, K - 1], bad[512, 0] = np.inf, np.nan, -np.inf
+    rows = [5, 300, 512]
+    for bf16 in (False, True):
+        ys = []
+        for v in (x, bad):
+            y = torch.empty(T, N, device="cuda")
+            if bf16:
+                xb = torch.from_numpy(O.f32_to_bf16(v).view(np.int16)).cuda()
+                ops.launch_gemm_bf16x(xb, W.view, None, T, K, N, y)
+            else:
+                ops.launch_gemm_tiled_q(torch.from_numpy(v).cuda(), W.view, None, T, K, N, y)
+            ys.append(y)
+        torch.cuda.synchronize()
+        keep = torch.ones(T, dtype=torch.bool, device="cuda")
+        keep[rows] = False
+        assert torch.equal(ys[0][keep], ys[1][keep])
+        assert not torch.isfinite(ys[1][rows]).all(1).any()
