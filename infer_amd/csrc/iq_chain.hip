@@ -509,38 +509,70 @@ __device__ __forceinline__ float block256_sum(float v, float* red4) {
     return ((red4[0] + red4[1]) + red4[2]) + red4[3];
 }
 
-// Output side of a B-row stage: thread (column c, row m = blockIdx.y).
-__global__ __launch_bounds__(256) void epi_kernel(const CEpi e) {
-    __shared__ float red4[4];
+// Output side of a B-row stage: one wave per 256 columns of row m =
+// blockIdx.y, four consecutive columns of a 16-column tile per thread.  The
+// bias and the residual are requested before the range sums.  (1.5B chain at
+// 24 sequences against a column per thread: the lm_head's sums 16.8 -> 10.2
+// us, the chain 511 -> 505.)
+__global__ __launch_bounds__(64) void epi_kernel(const CEpi e) {
     const int m = blockIdx.y;
-    const int c = int(blockIdx.x) * 256 + int(threadIdx.x);
+    const int c = (int(blockIdx.x) * 64 + int(threadIdx.x)) * 4;
     const int64_t stride = int64_t(e.M) * e.ld, base = int64_t(m) * e.ld;
-    float v = 0.0f;
-    bool valid = false;
+    float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
     if (c < e.ncols) {
+        // this thread's matrix (SwiGLU: the first, gate)
+        float* y = e.y[0];
+        const uint16_t* bias = e.bias[0];
+        int N = e.N[0], first = 0;
+#pragma unroll
+        for (int k = 1; k < kMaxStageMats; k++)
+            if (!e.swiglu && k < e.nmat && c >= e.tile0[k] * 16) {
+                y = e.y[k];
+                bias = e.bias[k];
+                N = e.N[k];
+                first = e.tile0[k] * 16;
+            }
+        const int col = c - first, n = N - col < 4 ? N - col : 4;  // columns of the matrix here
+        float* dst = y + int64_t(m) * N + col;
+        const float* res = e.res ? e.res + int64_t(m) * N + col : nullptr;
+        float b[4] = {}, b1[4] = {}, r[4] = {};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (k >= n) continue;
+            if (bias) b[k] = bf16_to_f32(bias[col + k]);
+            if (e.swiglu && e.bias[1]) b1[k] = bf16_to_f32(e.bias[1][col + k]);
+            if (res) r[k] = res[k];
+        }
+        v = sum_slices4(e.part, e.S, stride, base + c);
         if (e.swiglu) {
             // silu(g) * u  (kernels/ops/elementwise.cu:6-11)
-            const float g = sum_slices(e.part, e.S, stride, base + c) + (e.bias[0] ? bf16_to_f32(e.bias[0][c]) : 0.0f);
-            const float u = sum_slices(e.part, e.S, stride, base + int64_t(e.tile0[1]) * 16 + c) +
-                            (e.bias[1] ? bf16_to_f32(e.bias[1][c]) : 0.0f);
-            v = g / (1.0f + expf(-g)) * u;
-            e.y[0][int64_t(m) * e.N[0] + c] = v;
-            valid = true;
+            const float4_t u = sum_slices4(e.part, e.S, stride, base + int64_t(e.tile0[1]) * 16 + c);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float g = v[k] + b[k];
+                v[k] = g / (1.0f + expf(-g)) * (u[k] + b1[k]);
+            }
         } else {
-            int i = 0;
-            for (int k = 1; k < e.nmat; k++)
-                if (c >= e.tile0[k] * 16) i = k;
-            const int col = c - e.tile0[i] * 16;
-            if (col < e.N[i]) {
-                v = sum_slices(e.part, e.S, stride, base + c) + (e.bias[i] ? bf16_to_f32(e.bias[i][col]) : 0.0f);
-                if (e.res) v = e.res[int64_t(m) * e.N[0] + col] + v;
-                e.y[i][int64_t(m) * e.N[i] + col] = v;
-                valid = true;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = v[k] + b[k];
+                if (res) v[k] = r[k] + v[k];
+            }
+        }
+        if (n == 4 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+            *reinterpret_cast<float4_t*>(dst) = v;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (k < n) dst[k] = v[k];
+                else v[k] = 0.0f;
             }
         }
     }
-    if (e.ssq_out) {
-        const float sq = block256_sum(valid ? v * v : 0.0f, red4);
+    if (e.ssq_out) {  // (one 256-column block a wave)
+        float sq = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o, 64);
         if (threadIdx.x == 0) e.ssq_out[int64_t(m) * e.ssq_n + blockIdx.x] = sq;
     }
 }
@@ -568,7 +600,7 @@ hipError_t run_rows_stage(const HostStage& h, float* part, int64_t part_floats, 
     CEpi ep = h.epi;
     ep.part = part;
     ep.S = S;
-    epi_kernel<<<dim3(unsigned((ep.ncols + 255) / 256), unsigned(h.rows)), 256, 0, stream>>>(ep);
+    epi_kernel<<<dim3(unsigned((ep.ncols + 255) / 256), unsigned(h.rows)), 64, 0, stream>>>(ep);
     return hipGetLastError();
 }
 

@@ -888,20 +888,7 @@ __global__ __launch_bounds__(256) void gemm_reduce4_kernel(const float* __restri
                                                            float* __restrict__ y) {
     const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (i >= T * N) return;
-    const int64_t stride = T * N;
-    const rsrc_t r = make_rsrc(part, int64_t(S) * stride * 4);
-    float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < S; s0 += 8) {
-        float4_t v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t off = s0 + j < S ? uint32_t((int64_t(s0 + j) * stride + i) * 4) : kOob;
-            v[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (s0 + j < S) sum += v[j];
-    }
+    const float4_t sum = sum_slices4(part, S, T * N, i);
     const int64_t n = i % N;
     float4_t o;
 #pragma unroll

@@ -83,14 +83,11 @@ __device__ __forceinline__ void load_x8(const float* xr, int64_t c0, int64_t K, 
 // One wave per (row, 4 groups); 16 lanes (one DPP row) per group, 8 columns
 // per lane.
 template <bool PERM, bool VECX>
-__global__ __launch_bounds__(256) void xprep_kernel(const float* __restrict__ x, int M, int64_t K,
-                                                    int64_t G, int64_t quads,
-                                                    int8_t* __restrict__ xq, int4* __restrict__ meta) {
+__global__ __launch_bounds__(64) void xprep_kernel(const float* __restrict__ x, int M, int64_t K, int64_t G,
+                                                   int8_t* __restrict__ xq, int4* __restrict__ meta) {
     const int lane = threadIdx.x & 63;
-    const int64_t wave = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (wave >= int64_t(M) * quads) return;
-    const int m = int(wave / quads);
-    const int64_t g = (wave % quads) * 4 + (lane >> 4);
+    const int m = blockIdx.y;
+    const int64_t g = int64_t(blockIdx.x) * 4 + (lane >> 4);
     const bool gvalid = g < G;
     const int j = lane & 15;
     float v[8];
@@ -1015,19 +1012,34 @@ __global__ __launch_bounds__(512) void gemvt_kernel(const GemvParams p) {
 }
 
 // y_i[m, n] = sum over ranges s of part[s][m][16*tile0_i + n] (in range
-// order) + bias_i[n], for every matrix i of a gemvt launch in one grid
-// (thread i covers (m, tile row) over all matrices' tiles).
-__global__ __launch_bounds__(256) void gemvt_reduce_kernel(const GemvParams p) {
-    const int64_t ld = int64_t(p.ntiles) * 16;
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= int64_t(p.M) * ld) return;
-    const int m = int(i / ld);
-    const int64_t c = i - int64_t(m) * ld;
-    const TileSel ts = select_tile(p, int(c >> 4));
+// order) + bias_i[n], for every matrix i of a launch in one grid: row m =
+// blockIdx.y, four consecutive columns of a tile per thread.  Bound by the
+// latency of a launch and of ceil(S / 8) loads; the arithmetic around them
+// (a column and a 64-bit division per thread) cost too: with this form and
+// the preparation's grid over (row, groups) instead of divisions, 8 layers
+// of 7B int4 at 16 rows 638 -> 628 us.
+__global__ __launch_bounds__(128) void gemvt_reduce_kernel(const GemvParams p) {
+    const int ld = p.ntiles * 16, m = blockIdx.y;
+    const int c = (int(blockIdx.x) * 128 + int(threadIdx.x)) * 4;
+    if (c >= ld) return;
+    const TileSel ts = select_tile(p, c >> 4);
     const int64_t row = ts.row0 + (c & 15);
-    if (row >= ts.m.N) return;
-    const float sum = sum_slices(p.part, p.S, int64_t(p.M) * ld, int64_t(m) * ld + c);
-    ts.m.y[int64_t(m) * ts.m.N + row] = sum + (ts.m.bias ? bf16_to_f32(ts.m.bias[row]) : 0.0f);
+    float b[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) b[e] = ts.m.bias && row + e < ts.m.N ? bf16_to_f32(ts.m.bias[row + e]) : 0.0f;
+    const float4_t sum = sum_slices4(p.part, p.S, int64_t(p.M) * ld, int64_t(m) * ld + c);
+    float* dst = ts.m.y + int64_t(m) * ts.m.N + row;
+    if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0 && row + 3 < ts.m.N) {
+        *reinterpret_cast<float4_t*>(dst) = float4_t{sum[0] + b[0], sum[1] + b[1], sum[2] + b[2], sum[3] + b[3]};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (row + e < ts.m.N) dst[e] = sum[e] + b[e];
+    }
+}
+
+void launch_gemvt_reduce(const GemvParams& p, hipStream_t stream) {
+    gemvt_reduce_kernel<<<dim3(unsigned((p.ntiles * 4 + 127) / 128), unsigned(p.M)), 128, 0, stream>>>(p);
 }
 
 // y[m, n] = sum over slices s of part[s, m, n] (in slice order) + bias[n].
@@ -1304,7 +1316,7 @@ hipError_t launch_gemv1(const float* x, const QView* W, const uint16_t* const* b
     GemvParams pr = p;
     pr.S = pl.kr;
     const int64_t cnt = int64_t(M) * tiles * 16;
-    gemvt_reduce_kernel<<<unsigned((cnt + 255) / 256), 256, 0, stream>>>(pr);
+    launch_gemvt_reduce(pr, stream);
     return hipGetLastError();
 }
 
@@ -1317,16 +1329,14 @@ int total_tiles(const QView* W, int n) {
 // Byte limbs + meta of x [M][K] into the workspace.
 hipError_t launch_xprep_limbs(const float* x, int M, int64_t K, int kind, Workspace* ws, hipStream_t stream) {
     const int64_t G = (K + kGroup - 1) / kGroup;
-    const int64_t quads = (G + 3) / 4;
-    const int64_t waves = int64_t(M) * quads;
-    const unsigned grid = unsigned((waves + 3) / 4);
+    const dim3 grid(unsigned((G + 3) / 4), unsigned(M));  // (4 groups, row)
     const bool vecx = (K % 4 == 0) && (reinterpret_cast<uintptr_t>(x) % 16 == 0);
     if (kind == 1) {
-        if (vecx) xprep_kernel<true, true><<<grid, 256, 0, stream>>>(x, M, K, G, quads, ws->xq, ws->xmeta);
-        else xprep_kernel<true, false><<<grid, 256, 0, stream>>>(x, M, K, G, quads, ws->xq, ws->xmeta);
+        if (vecx) xprep_kernel<true, true><<<grid, 64, 0, stream>>>(x, M, K, G, ws->xq, ws->xmeta);
+        else xprep_kernel<true, false><<<grid, 64, 0, stream>>>(x, M, K, G, ws->xq, ws->xmeta);
     } else {
-        if (vecx) xprep_kernel<false, true><<<grid, 256, 0, stream>>>(x, M, K, G, quads, ws->xq, ws->xmeta);
-        else xprep_kernel<false, false><<<grid, 256, 0, stream>>>(x, M, K, G, quads, ws->xq, ws->xmeta);
+        if (vecx) xprep_kernel<false, true><<<grid, 64, 0, stream>>>(x, M, K, G, ws->xq, ws->xmeta);
+        else xprep_kernel<false, false><<<grid, 64, 0, stream>>>(x, M, K, G, ws->xq, ws->xmeta);
     }
     return hipGetLastError();
 }
@@ -1460,7 +1470,7 @@ bool launch_gemvt(const QView* W, const uint16_t* const* bias, float* const* y, 
         else launch_gemvt_k<0>(p, pl, stream);
         if (pl.ks > 1) {
             const int64_t cnt = int64_t(mb) * tiles * 16;
-            gemvt_reduce_kernel<<<unsigned((cnt + 255) / 256), 256, 0, stream>>>(p);
+            launch_gemvt_reduce(p, stream);
         }
         *err = hipGetLastError();
         if (*err != hipSuccess) return true;
@@ -1494,43 +1504,34 @@ constexpr int kHGroupBytes = 4 * 2 * 64 * 16;  // prepared bytes per (block, gro
 // weights); fac: 2^-k, or NaN when the group holds a non-finite value.
 template <bool PERM>
 __device__ __forceinline__ void xh_split8(const float (&v)[8], half8_t& ho, half8_t& lo, float& fac) {
-    // largest |x| bits over the 16 lanes; a NaN or an infinity has larger
-    // bits (>= 0x7F800000) than any finite value, so one test of the
-    // maximum finds any of them
-    uint32_t am = 0;
+    // largest |x| over the 16 lanes (max ignores a NaN; an infinity stays)
+    float am = __builtin_fabsf(v[0]);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const uint32_t a = __float_as_uint(v[i]) & 0x7FFFFFFFu;
-        am = a > am ? a : am;
-    }
-    am = row16_max_u32(am);
-    const bool fin = am < 0x7F800000u;
+    for (int i = 1; i < 8; i++) am = __builtin_fmaxf(am, __builtin_fabsf(v[i]));
+    am = row16_max(am);
     // amax = f 2^E, f in [0.5, 1): k = 15 - E puts amax 2^k in [2^14, 2^15)
-    const int k = (am > 0 && fin) ? 15 - __builtin_amdgcn_frexp_expf(__uint_as_float(am)) : 0;
-    // operand dword j: values (j, j + 4) with PERM, else (2j, 2j + 1).
-    // (A group with a non-finite value keeps its values: fac is NaN, so its
-    // row's outputs are NaN whatever the operand holds, and an MFMA output
-    // row reads only its own operand row.)
+    // (frexp's exponent of 0, infinity and NaN is 0)
+    const int k = am > 0.0f ? 15 - __builtin_amdgcn_frexp_expf(am) : 0;
+    // operand dword j: values (j, j + 4) with PERM, else (2j, 2j + 1).  The
+    // residual s - hi is exact (one v_fma_mix each).  A non-finite value
+    // needs no care: hi or lo of it is NaN, so its row's products are (an
+    // MFMA output row reads only its own operand row).
+    float m1;  // (in a register the compiler cannot see into: a product
+               // with a visible -1 becomes a conversion and a subtraction)
+    asm("s_mov_b32 %0, -1.0" : "=s"(m1));
     u32x4_t hw, lw;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int e0 = PERM ? j : 2 * j, e1 = PERM ? j + 4 : 2 * j + 1;
-        const float s0 = __builtin_amdgcn_ldexpf(v[e0], k);
-        const float s1 = __builtin_amdgcn_ldexpf(v[e1], k);
-        half2_t h, l;
-        h[0] = _Float16(s0);
-        h[1] = _Float16(s1);
-        const uint32_t hb = h2_bits(h);
-        const float b0 = float(__builtin_bit_cast(_Float16, uint16_t(hb)));
-        const float b1 = float(__builtin_bit_cast(_Float16, uint16_t(hb >> 16)));
-        l[0] = _Float16(s0 - b0);
-        l[1] = _Float16(s1 - b1);
-        hw[j] = hb;
-        lw[j] = h2_bits(l);
+        const float2_t s = {__builtin_amdgcn_ldexpf(v[e0], k), __builtin_amdgcn_ldexpf(v[e1], k)};
+        const half2_t h = __builtin_convertvector(s, half2_t);
+        const float2_t r = {__builtin_fmaf(float(h[0]), m1, s[0]), __builtin_fmaf(float(h[1]), m1, s[1])};
+        hw[j] = h2_bits(h);
+        lw[j] = h2_bits(__builtin_convertvector(r, half2_t));
     }
     ho = __builtin_bit_cast(half8_t, hw);
     lo = __builtin_bit_cast(half8_t, lw);
-    fac = fin ? __builtin_amdgcn_ldexpf(1.0f, -k) : __builtin_nanf("");
+    fac = __builtin_amdgcn_ldexpf(1.0f, -k);
 }
 
 // PK (M <= 8): one A operand per k-chunk holds both terms, rows 0..7 the hi
@@ -1538,14 +1539,11 @@ __device__ __forceinline__ void xh_split8(const float (&v)[8], half8_t& ho, half
 // half the operand bytes and MFMAs); the kernel adds the two halves of each
 // output at the end.
 template <bool PERM, bool PK>
-__global__ __launch_bounds__(256) void xhprep_kernel(const float* __restrict__ x, int M, int64_t K, int64_t G,
-                                                     int64_t quads, int nb, _Float16* __restrict__ xh,
-                                                     float* __restrict__ xfx) {
+__global__ __launch_bounds__(64) void xhprep_kernel(const float* __restrict__ x, int M, int64_t K, int64_t G,
+                                                     _Float16* __restrict__ xh, float* __restrict__ xfx) {
     const int lane = threadIdx.x & 63, j16 = lane & 15;
-    const int64_t wave = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (wave >= int64_t(nb) * 16 * quads) return;
-    const int m = int(wave / quads);  // 0 .. 16 nb - 1 (rows past M are written as zeros)
-    const int64_t g = (wave % quads) * 4 + (lane >> 4);
+    const int m = blockIdx.y;  // rows past M are written as zeros
+    const int64_t g = int64_t(blockIdx.x) * 4 + (lane >> 4);
     const bool gvalid = g < G;
     float v[8];
     load_x8<1>(x + int64_t(m < M ? m : 0) * K, (gvalid && m < M ? g : 0) * kGroup + j16 * 8,
@@ -1577,15 +1575,13 @@ __global__ __launch_bounds__(256) void xhprep_kernel(const float* __restrict__ x
 // multiplies the group factor by it after the split, so the operands and
 // factors equal those the prologue instances make.
 template <bool PERM>
-__global__ __launch_bounds__(256) void xhprep_pro_kernel(const GemvParams p, int64_t quads, int nb,
-                                                         _Float16* __restrict__ xh, float* __restrict__ xfx) {
+__global__ __launch_bounds__(64) void xhprep_pro_kernel(const GemvParams p, _Float16* __restrict__ xh,
+                                                         float* __restrict__ xfx) {
     const int lane = threadIdx.x & 63, j16 = lane & 15;
-    const int64_t wave = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (wave >= int64_t(nb) * 16 * quads) return;
     const int M = p.M;
     const int64_t G = p.G;
-    const int m = int(wave / quads);  // rows past M are written as zeros
-    const int64_t g = (wave % quads) * 4 + (lane >> 4);
+    const int m = blockIdx.y;  // rows past M are written as zeros
+    const int64_t g = int64_t(blockIdx.x) * 4 + (lane >> 4);
     const bool ok = g < G && m < M;
     const int64_t c = (ok ? g : 0) * kGroup + j16 * 8;
     const rsrc_t rx = make_rsrc(p.x, int64_t(M) * p.xstride * 4);
@@ -2329,6 +2325,335 @@ __global__ __launch_bounds__(512, (PRO && (LOOP || (KIND == 0 && MB == 2))) ? 2 
     }
 }
 
+// 5..32 rows, each wave keeping its share of the activations in registers:
+// wave w of a workgroup takes NG groups of K (the workgroup's nw waves a
+// range of gs = nw NG groups, at most 32 at up to 16 rows and 16 at 17..32)
+// and walks the workgroup's 16-row tiles over them, its f16 split operands
+// made once, in registers (through the wave's own LDS, no barrier), and the
+// next D tiles' weights, scales and zero points in flight; the waves' sums
+// of CH tiles are added from LDS in wave order.  One workgroup of up to 8
+// waves per CU, the tiles dealt out evenly, so the weights stream from the
+// first to the last instruction; rows of up to 32 (16) groups need no range
+// sums and no reduction launch, and no call needs a preparation launch.
+// The kernels that made a short K range's operands per workgroup and loaded
+// everything at once (gemvr, gemvq) spent their time starting and draining,
+// and on the range sums.  hi and lo products are summed apart (the error
+// against 64 bits is no larger than theirs: 8.5e-8 on 7B gate|up).
+// Measured (one MI355X, in a graph, us): 7B int4 at 16 rows gate|up 32.6 ->
+// 26.1, down 23.8 -> 21.9, q|k|v 12.3 -> 11.5; int8 at 5 rows gate|up 37.7
+// -> 30.3, down 25.0 -> 23.6; at 32 rows gate|up 62.0 -> 43.3, down 36.9 ->
+// 28.2, lm_head 171 -> 139; 1.5B gate|up int4 at 24 rows 18.5 -> 15.2.
+// MB2 (half blocks): 1 for up to 8 rows (packed: rows 0..7 of an operand
+// the hi, 8..15 the lo terms), 2 for up to 16, 4 for up to 32 rows.  D = 2:
+// with 3 tiles in flight the 16-row int4 instance spills (gate|up 30.2 us),
+// with 4 the others gain nothing.
+template <int KIND, int MB2, int NG>
+struct GwShape {
+    static constexpr int ROWS = 8 * MB2;                       // activation rows held
+    static constexpr int BLK = MB2 == 4 ? 2 : 1;               // 16-row operand blocks
+    static constexpr int OPS = MB2 == 1 ? 4 : 8;               // operands per group and block
+    static constexpr int NX = ROWS * NG * 16 / 64;             // 8-value tasks per lane
+    static constexpr int D = 2;                                // tiles requested ahead
+    static constexpr int CH = 4;                               // tiles between two sums over the waves
+    static constexpr int CS = 65;                              // 16-byte slots between operands in LDS
+    static constexpr int OPB = OPS * CS * 16;                  // bytes of a (group, block)'s operands
+    static constexpr int PARTB = 2 * CH * 64 * 16 * BLK;       // bytes of a wave's partial sums
+    static constexpr int FACB = NG * BLK * 64;                 // bytes of the group factors
+    static constexpr int WAVEB = (OPB > PARTB ? OPB : PARTB) + FACB;
+};
+
+template <int KIND, int MB2, int NG>
+__global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
+    using S = GwShape<KIND, MB2, NG>;
+    constexpr bool PK = MB2 == 1;
+    constexpr int WPG = KIND == 1 ? 1 : 2;
+    extern __shared__ __attribute__((aligned(16))) int8_t wlds[];
+    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = int(blockDim.x) >> 6;
+    const int G = int(p.G);
+    const int rb = int(blockIdx.x) % p.nrb, range = int(blockIdx.x) / p.nrb;
+    const int g0 = range * p.gs + wave * NG;
+    const int gend = range * p.gs + p.gs < G ? range * p.gs + p.gs : G;
+    const int ng = gend - g0 < 0 ? 0 : (gend - g0 < NG ? gend - g0 : NG);
+    const int t0 = int(int64_t(rb) * p.ntiles / p.nrb), t1 = int(int64_t(rb + 1) * p.ntiles / p.nrb);
+    const int row_bytes = int(KIND == 1 ? p.K / 2 : p.K);
+    int8_t* const mine = wlds + wave * S::WAVEB;
+
+    // 1. this wave's activations: its groups of every row
+    float xv[S::NX][8];
+    {
+        const rsrc_t rxx = make_rsrc(p.x, int64_t(p.M) * p.K * 4);
+#pragma unroll
+        for (int u = 0; u < S::NX; u++) {
+            const int t = lane + 64 * u, pr = t >> 4;
+            const int m = pr % S::ROWS, i = pr / S::ROWS;
+            const uint32_t o = (i < ng && m < p.M) ? uint32_t((int64_t(m) * p.K + int64_t(g0 + i) * kGroup + ln * 8) * 4) : kOob;
+            const float4_t a = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rxx, o, 0, 0));
+            const float4_t b = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rxx, o, 16, 0));
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                xv[u][e] = a[e];
+                xv[u][4 + e] = b[e];
+            }
+        }
+    }
+    // 2. the first tiles' weights, scales and zero points
+    struct Buf {
+        int4v_t w[NG][WPG];
+        uint32_t s[NG / 2];  // bf16 scales, two a word
+        uint32_t z;          // zero points, one a byte
+    };
+    Buf bufs[S::D];
+    auto request = [&](Buf& b, int tile) {
+        const bool ok = tile < t1;
+        const TileSel ts = select_tile(p, ok ? tile : t0);
+        const int64_t left = ts.m.N - ts.row0;
+        const int64_t rows = ok ? (left < 16 ? left : 16) : 0;
+        const rsrc_t rq = make_rsrc_wave(ts.m.q + ts.row0 * row_bytes, rows * row_bytes);
+        const rsrc_t rs = make_rsrc_wave(ts.m.scales + ts.row0 * G, rows * G * 2);
+        const rsrc_t rz = make_rsrc_wave(KIND == 1 ? ts.m.zeros + ts.row0 * G : nullptr, KIND == 1 ? rows * G : 0);
+        const uint32_t vq = uint32_t(ln * row_bytes + q * (KIND == 1 ? 16 : 32));
+        // (G % NG == 0: a wave's groups are all there or none is)
+        const uint32_t vs = uint32_t(ln * G) + (ng > 0 ? 0u : kOob / 2);
+        if (NG == 4) {
+            const uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, vs * 2, g0 * 2, 0));
+            b.s[0] = v.x;
+            b.s[NG / 2 - 1] = v.y;
+            b.z = KIND == 1 ? uint32_t(__builtin_amdgcn_raw_buffer_load_b32(rz, vs, g0, 0)) : 0u;
+        } else {
+            b.s[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, vs * 2, g0 * 2, 0);
+            b.z = KIND == 1 ? uint32_t(__builtin_amdgcn_raw_buffer_load_b16(rz, vs, g0, 0)) : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < NG; i++) {
+            const uint32_t o = i < ng ? 0u : kOob;
+#pragma unroll
+            for (int h = 0; h < WPG; h++)
+                b.w[i][h] = __builtin_bit_cast(int4v_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                           rq, vq + o, (g0 + i) * (KIND == 1 ? 64 : 128) + h * 16, 0));
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < S::D; d++) request(bufs[d], t0 + d);
+    // 3. the operands, group by group through the wave's own LDS
+    half8_t ops[NG][S::BLK][S::OPS];
+#pragma unroll
+    for (int i = 0; i < NG; i++) {
+#pragma unroll
+        for (int b = 0; b < S::BLK; b++) {
+            half8_t* dst = reinterpret_cast<half8_t*>(mine);
+            float* fs = reinterpret_cast<float*>(mine + S::WAVEB - S::FACB) + (i * S::BLK + b) * 16;
+            constexpr int TB = S::NX / NG / S::BLK;  // tasks of a (group, block)
+#pragma unroll
+            for (int u = 0; u < TB; u++) {
+                const int m = (lane >> 4) + 4 * u;  // row in the block
+                half8_t ho, lo;
+                float fac;
+                xh_split8<KIND == 1>(xv[(i * S::BLK + b) * TB + u], ho, lo, fac);
+                const int qq = ln >> 2, jj = ln & 3;
+                if (PK) {
+                    dst[jj * S::CS + m + 16 * qq] = ho;
+                    dst[jj * S::CS + m + 8 + 16 * qq] = lo;
+                } else {
+                    dst[(jj * 2) * S::CS + m + 16 * qq] = ho;
+                    dst[(jj * 2 + 1) * S::CS + m + 16 * qq] = lo;
+                }
+                if (ln == 0) fs[m] = fac;
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int o = 0; o < S::OPS; o++) ops[i][b][o] = dst[o * S::CS + lane];
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    // 4. the tiles
+    auto multiply = [&](Buf& bf, float4_t* slot) {
+        // (the group factors stay in LDS: in registers they would push out a
+        // tile's weights)
+        const float4_t* const fac = reinterpret_cast<const float4_t*>(mine + S::WAVEB - S::FACB) + (PK ? q & 1 : q);
+        float4_t acc[S::BLK];
+#pragma unroll
+        for (int b = 0; b < S::BLK; b++) acc[b] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < NG; i++) {
+            half8_t B[4];
+            if (KIND == 1) {
+                const uint32_t z = (bf.z >> (8 * i)) & 0xFFu;
+                const uint32_t zb = zpair_1024(z), zc = zpair_64(z);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    uint32_t o0, o1, o2, o3;
+                    dq_int4_x8(uint32_t(bf.w[i][0][j]), zb, zc, o0, o1, o2, o3);
+                    B[j] = pack_h8(o0, o1, o2, o3);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    uint32_t l0, h0, l1, h1;
+                    const int4v_t& w = bf.w[i][KIND == 1 ? 0 : j >> 1];
+                    dq_int8_x4(uint32_t(w[2 * (j & 1)]), l0, h0);
+                    dq_int8_x4(uint32_t(w[2 * (j & 1) + 1]), l1, h1);
+                    B[j] = pack_h8(l0, h0, l1, h1);
+                }
+            }
+            const float sc = __uint_as_float((i & 1) ? (bf.s[i >> 1] & 0xFFFF0000u) : (bf.s[i >> 1] << 16));
+#pragma unroll
+            for (int b = 0; b < S::BLK; b++) {
+                // the hi and lo products summed apart
+                const float4_t fx = fac[(i * S::BLK + b) * 4];
+                float4_t P = {0.0f, 0.0f, 0.0f, 0.0f}, Q = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (PK) {
+                        P = mfma16(ops[i][b][j], B[j], P);
+                    } else {
+                        P = mfma16(ops[i][b][2 * j], B[j], P);
+                        Q = mfma16(ops[i][b][2 * j + 1 < S::OPS ? 2 * j + 1 : 0], B[j], Q);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    acc[b][r] = __builtin_fmaf(PK ? P[r] : P[r] + Q[r], sc * fx[r], acc[b][r]);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < S::BLK; b++) slot[b * 64 + lane] = acc[b];
+    };
+    // the waves' sums of tiles [c, c + n), in wave order
+    auto finish = [&](int c, int n, int odd) {
+        for (int it = wave; it < n * S::BLK; it += nw) {
+            const int b = it % S::BLK, tile = c + it / S::BLK;
+            const float4_t* src = reinterpret_cast<const float4_t*>(wlds) + odd * (S::CH * 64 * S::BLK) + it * 64 + lane;
+            float4_t sum = src[0];
+            for (int w = 1; w < nw; w++) sum += src[w * (S::WAVEB / 16)];
+            if (PK) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[r] += __shfl_down(sum[r], 32, 64);
+            }
+            const TileSel ts = select_tile(p, tile);
+            const int64_t row = ts.row0 + ln;
+            if (row >= ts.m.N || (PK && q >= 2)) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = 16 * b + 4 * q + r;
+                if (m >= p.M) continue;
+                if (p.S == 1) ts.m.y[int64_t(m) * ts.m.N + row] = sum[r] + (ts.m.bias ? bf16_to_f32(ts.m.bias[row]) : 0.0f);
+                else p.part[(int64_t(range) * p.M + m) * (int64_t(p.ntiles) * 16) + int64_t(tile) * 16 + ln] = sum[r];
+            }
+        }
+    };
+    int odd = 0, c = t0;
+    float4_t* const slots = reinterpret_cast<float4_t*>(mine);
+    for (; c + S::CH <= t1; c += S::CH, odd ^= 1) {
+#pragma unroll
+        for (int tt = 0; tt < S::CH; tt++) {
+            multiply(bufs[tt % S::D], slots + (odd * S::CH + tt) * 64 * S::BLK);
+            request(bufs[tt % S::D], c + tt + S::D);
+        }
+        __syncthreads();
+        finish(c, S::CH, odd);
+    }
+    if (c == t1) return;
+    // the last tiles, fewer than CH (all of theirs below D are requested)
+#pragma unroll
+    for (int tt = 0; tt < S::CH - 1; tt++) {
+        if (c + tt >= t1) break;
+        multiply(bufs[tt % S::D], slots + (odd * S::CH + tt) * 64 * S::BLK);
+        if (tt + S::D < S::CH - 1) request(bufs[tt % S::D], c + tt + S::D);
+    }
+    __syncthreads();
+    finish(c, t1 - c, odd);
+}
+
+template <int KIND, int MB2, int NG>
+void launch_gemvw_t(const GemvParams& p, unsigned grid, int nw, hipStream_t stream) {
+    const size_t lds = size_t(nw) * GwShape<KIND, MB2, NG>::WAVEB;
+    allow_big_lds<gemvw_kernel<KIND, MB2, NG>>();
+    gemvw_kernel<KIND, MB2, NG><<<grid, unsigned(64 * nw), lds, stream>>>(p);
+}
+
+// gemvw or the other kernels (both measured in a graph, us, others -> gemvw):
+// 17..32 rows from 64 tiles on (7B k 512 x 3584 at 17 rows 11.2 kept against
+// 11.4; 1024 x 7168 16.9 -> 12.6); 9..16 rows on long rows (1.5B down, G =
+// 70, int8 20.9 -> 11.0, int4 15.2 -> 10.2) or where tiles x groups fill the
+// card (7B q|k|v, 288 x 28, 12.3 -> 11.4; o, 224 x 28, int4 9.7 kept against
+// 10.4, int8 11.9 -> 11.1; 7168 x 1024, 448 x 8, 7.6 kept against 8.9); 5..8
+// rows wherever the 1-row kernel's exact integer sums do not serve (on those
+// narrow calls, where gemvw would be up to 25 % faster at 8 rows, its error
+// is 1.2 to 1.4 times theirs).
+bool gemvw_preferred(int M, int tiles, int64_t K, int kind) {
+    const int64_t G = K / kGroup;
+    if (M < 5 || M > kMaxRowsGemv || K % kGroup || G % 2) return false;
+    if (M > 16) return tiles >= 64;
+    if (M > 8) return G >= 48 || tiles * G >= (kind == 1 ? 6400 : 6000);
+    return tiles >= 1024 || G >= 128 || !gemv1_rows_preferred(M, tiles, G);
+}
+
+// gemvw on n matrices straight from x (false: G has no whole sets of
+// groups, or the partial sums would not fit).
+bool launch_gemvw(const float* x, const QView* W, const uint16_t* const* bias, float* const* y, int n, int M, Workspace* ws,
+                  hipStream_t stream, hipError_t* err) {
+    const int64_t K = W[0].cols, G = W[0].groups;
+    GemvParams p{};
+    int tiles = 0;
+    for (int i = 0; i < n; i++) {
+        p.mat[i] = MatRef{W[i].q, W[i].scales, W[i].zeros, bias[i], y[i], W[i].rows, tiles};
+        tiles += int((W[i].rows + 15) / 16);
+    }
+    // groups a wave: 4 (2 from 17 rows: their operands fill the registers),
+    // or 2 where G leaves a remainder; whole sets only
+    const int ng = M <= 16 && G % 4 == 0 ? 4 : 2;
+    if (G % ng) return false;
+    int S = int((G + 8 * ng - 1) / (8 * ng));
+    int gs = int((G + S - 1) / S);
+    gs = (gs + ng - 1) / ng * ng;
+    S = int((G + gs - 1) / gs);
+    const int nw = gs / ng;
+    if (S > 1 && int64_t(S) * M * tiles * 16 > ws->part_floats) return false;
+    const int slots = device_cu_count() * (8 / nw);
+    p.nmat = n;
+    p.K = K;
+    p.G = G;
+    p.x = x;
+    p.M = M;
+    p.gs = gs;
+    p.S = S;
+    p.ntiles = tiles;
+    p.nrb = std::min(tiles, std::max(1, slots / S));
+    if (tiles < 2 * p.nrb && tiles > p.nrb) p.nrb = (tiles + 1) / 2;
+    p.part = ws->partials;
+    const unsigned grid = unsigned(p.nrb * S);
+    const bool i4 = W[0].kind == 1;
+    if (M > 16) {
+        if (i4) launch_gemvw_t<1, 4, 2>(p, grid, nw, stream);
+        else launch_gemvw_t<0, 4, 2>(p, grid, nw, stream);
+    } else if (M > 8) {
+        if (ng == 4) {
+            if (i4) launch_gemvw_t<1, 2, 4>(p, grid, nw, stream);
+            else launch_gemvw_t<0, 2, 4>(p, grid, nw, stream);
+        } else {
+            if (i4) launch_gemvw_t<1, 2, 2>(p, grid, nw, stream);
+            else launch_gemvw_t<0, 2, 2>(p, grid, nw, stream);
+        }
+    } else {
+        if (ng == 4) {
+            if (i4) launch_gemvw_t<1, 1, 4>(p, grid, nw, stream);
+            else launch_gemvw_t<0, 1, 4>(p, grid, nw, stream);
+        } else {
+            if (i4) launch_gemvw_t<1, 1, 2>(p, grid, nw, stream);
+            else launch_gemvw_t<0, 1, 2>(p, grid, nw, stream);
+        }
+    }
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && S > 1) {
+        const int64_t outs = int64_t(M) * tiles * 16;
+        launch_gemvt_reduce(p, stream);
+        e = hipGetLastError();
+    }
+    *err = e;
+    return true;
+}
+
 // gemvr on n matrices, M in 5..16, straight from x (false: the partial sums
 // would not fit).
 bool launch_gemvr(const float* x, const QView* W, const uint16_t* const* bias, float* const* y, int n, int M, Workspace* ws,
@@ -2370,7 +2695,7 @@ bool launch_gemvr(const float* x, const QView* W, const uint16_t* const* bias, f
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
         const int64_t outs = int64_t(M) * tiles * 16;
-        gemvt_reduce_kernel<<<unsigned((outs + 255) / 256), 256, 0, stream>>>(p);
+        launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
     *err = e;
@@ -2441,7 +2766,7 @@ bool launch_gemvq(const float* x, const QView* W, const uint16_t* const* bias, f
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
         const int64_t outs = int64_t(M) * tiles * 16;
-        gemvt_reduce_kernel<<<unsigned((outs + 255) / 256), 256, 0, stream>>>(p);
+        launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
     *err = e;
@@ -2483,7 +2808,7 @@ bool launch_gemvs(const QView* W, const uint16_t* const* bias, float* const* y, 
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
         const int64_t outs = int64_t(M) * tiles * 16;
-        gemvt_reduce_kernel<<<unsigned((outs + 255) / 256), 256, 0, stream>>>(p);
+        launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
     *err = e;
@@ -2495,18 +2820,17 @@ bool launch_gemvs(const QView* W, const uint16_t* const* bias, float* const* y, 
 // gemvs reads).
 hipError_t launch_xhprep(const float* x, int M, int64_t K, int kind, Workspace* ws, hipStream_t stream,
                          bool pk = true) {
-    const int64_t G = K / kGroup, quads = (G + 3) / 4;
-    const int nb = (M + 15) / 16;
-    const int64_t waves = int64_t(nb) * 16 * quads;
-    const unsigned grid = unsigned((waves + 3) / 4);
+    const int64_t G = K / kGroup;
+    const bool packed = M <= 8 && pk;
+    const dim3 grid(unsigned((G + 3) / 4), unsigned(packed ? 8 : (M + 15) / 16 * 16));  // (4 groups, row)
     _Float16* xh = reinterpret_cast<_Float16*>(ws->xq);
     float* xfx = reinterpret_cast<float*>(ws->xmeta);
-    if (M <= 8 && pk) {
-        if (kind == 1) xhprep_kernel<true, true><<<grid, 256, 0, stream>>>(x, M, K, G, quads, nb, xh, xfx);
-        else xhprep_kernel<false, true><<<grid, 256, 0, stream>>>(x, M, K, G, quads, nb, xh, xfx);
+    if (packed) {
+        if (kind == 1) xhprep_kernel<true, true><<<grid, 64, 0, stream>>>(x, M, K, G, xh, xfx);
+        else xhprep_kernel<false, true><<<grid, 64, 0, stream>>>(x, M, K, G, xh, xfx);
     } else {
-        if (kind == 1) xhprep_kernel<true, false><<<grid, 256, 0, stream>>>(x, M, K, G, quads, nb, xh, xfx);
-        else xhprep_kernel<false, false><<<grid, 256, 0, stream>>>(x, M, K, G, quads, nb, xh, xfx);
+        if (kind == 1) xhprep_kernel<true, false><<<grid, 64, 0, stream>>>(x, M, K, G, xh, xfx);
+        else xhprep_kernel<false, false><<<grid, 64, 0, stream>>>(x, M, K, G, xh, xfx);
     }
     return hipGetLastError();
 }
@@ -2671,6 +2995,18 @@ hipError_t launch_gemv_prepped(const QView& W, const uint16_t* bias, int M, floa
 hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* const* bias, float* const* y,
                              int n, int M, Workspace* ws, hipStream_t stream) {
     const int64_t K = W[0].cols, G = W[0].groups;
+    if (gemvw_preferred(M, total_tiles(W, n), K, W[0].kind)) {
+        hipError_t e = hipSuccess;
+        if (launch_gemvw(x, W, bias, y, n, M, ws, stream, &e)) {
+            // gemvw leaves a preparation's buffers alone, but callers may
+            // rely on the refusal that the kernels before it on these calls
+            // gave iq_gemv_prepped by reusing them
+            const int tiles = total_tiles(W, n);
+            const bool forget = M > 8 ? M <= 16 : (tiles < 1024 && G < 128) || (W[0].kind == 0 && M >= 7 && tiles >= 4096);
+            if (forget && !ws->prep_copy) ws->invalidate_prep();
+            return e;
+        }
+    }
     if (gemvq_rows_preferred(M, total_tiles(W, n), K, n)) {
         hipError_t e = hipSuccess;
         if (launch_gemvq(x, W, bias, y, n, M, ws, stream, &e)) return e;
@@ -2797,7 +3133,11 @@ hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* con
 
 bool launch_gemm_rows(const float* x, const QView& W, const uint16_t* bias, int64_t T, float* y, Workspace* ws,
                       hipStream_t stream, hipError_t* err) {
-    if (!gemvq_rows_preferred(T, int((W.rows + 15) / 16), W.cols, 1)) return false;
+    const int tiles = int((W.rows + 15) / 16);
+    if (T > 16 && T <= kMaxRowsGemv && gemvw_preferred(int(T), tiles, W.cols, W.kind) &&
+        launch_gemvw(x, &W, &bias, &y, 1, int(T), ws, stream, err))
+        return true;
+    if (!gemvq_rows_preferred(T, tiles, W.cols, 1)) return false;
     return launch_gemvq(x, &W, &bias, &y, 1, int(T), ws, stream, err);
 }
 
@@ -2951,7 +3291,7 @@ hipError_t launch_chain_h(const QView* W, int n, int M, const RowsIn& in, const 
                           float* const* y, const float* res, float* ssq_out, int8_t* xq, float* xmeta,
                           hipStream_t stream) {
     if (!chain_h_applies(W, n, M)) return hipErrorInvalidValue;
-    const int64_t K = W[0].cols, G = W[0].groups, quads = (G + 3) / 4;
+    const int64_t K = W[0].cols, G = W[0].groups;
     const int nb = (M + 15) / 16;
     GemvParams pp{};
     pp.x = in.x;
@@ -2965,10 +3305,10 @@ hipError_t launch_chain_h(const QView* W, int n, int M, const RowsIn& in, const 
     pp.M = M;
     pp.K = K;
     pp.G = G;
-    const unsigned grid = unsigned((int64_t(nb) * 16 * quads + 3) / 4);
+    const dim3 grid(unsigned((G + 3) / 4), unsigned(nb * 16));  // (4 groups, row)
     _Float16* xh = reinterpret_cast<_Float16*>(xq);
-    if (W[0].kind == 1) xhprep_pro_kernel<true><<<grid, 256, 0, stream>>>(pp, quads, nb, xh, xmeta);
-    else xhprep_pro_kernel<false><<<grid, 256, 0, stream>>>(pp, quads, nb, xh, xmeta);
+    if (W[0].kind == 1) xhprep_pro_kernel<true><<<grid, 64, 0, stream>>>(pp, xh, xmeta);
+    else xhprep_pro_kernel<false><<<grid, 64, 0, stream>>>(pp, xh, xmeta);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // (the unpacked operand form at 5..8 rows too: rows 8..15 of each block

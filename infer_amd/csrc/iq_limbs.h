@@ -231,4 +231,23 @@ __device__ __forceinline__ float sum_slices(const float* part, int S, int64_t st
     return sum;
 }
 
+// The same for the four consecutive sums i .. i + 3 (stride and i multiples
+// of 4, part 16-byte aligned): one 16-byte request per slice.
+__device__ __forceinline__ float4_t sum_slices4(const float* part, int S, int64_t stride, int64_t i) {
+    const rsrc_t r = make_rsrc(part, int64_t(S) * stride * 4);
+    float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < S; s0 += 8) {
+        float4_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t off = s0 + j < S ? uint32_t((int64_t(s0 + j) * stride + i) * 4) : kOob;
+            v[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (s0 + j < S) sum += v[j];
+    }
+    return sum;
+}
+
 }  // namespace iq
