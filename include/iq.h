@@ -159,8 +159,8 @@ int iq_quantize(const uint16_t* w_bf16, int64_t rows, int64_t cols, int kind, ui
  * GpuBatch::Impl::launch_sequence (kernels/batch_gpu.cu:186-215), each
  * stage reading what earlier stages wrote, with the elementwise work
  * between them fused into the stages.  A run is one launch per 1-row stage
- * and two per B-row stage (the GEMV with the input transform, then the
- * K-range sums with the output transform), on one stream, capturable into
+ * and one or two per B-row stage (the GEMV with the input transform, and on
+ * long rows the K-range sums with the output transform), on one stream, capturable into
  * a HIP graph.  No reference counterpart as an entry point: the reference
  * issues launch_gemv_batched_q, launch_rmsnorm, launch_swiglu and
  * launch_residual_add separately.

@@ -121,6 +121,7 @@ struct HostStage {
     // B-row stages (rows > 1)
     int rows = 1;
     int fused_r = 1;  // > 1: one stage_kernel launch of the R-row instance (rows <= R)
+    bool wroute = false;  // B rows on rows of few groups: one gemvw launch (no epilogue launch)
     bool hroute = false;  // B rows on a narrow stage: operand preparation + gemvh (no epilogue launch)
     QView W[kMaxStageMats];
     RowsIn in{};
@@ -811,10 +812,16 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
             ep.swiglu = pair ? 1 : 0;
             ep.res = a.out_op == IQ_OUT_RESIDUAL ? a.residual : nullptr;
             ep.ncols = pair ? int32_t(W0.rows) : int32_t(ep.ld);
-            // narrow stages (q|k|v, o at 9..32 rows): the input transform
-            // into prepared f16 operands, then gemvh with bias, residual and
-            // per-tile sums of squares in its own epilogue
-            hs.hroute = !pair && (a.out_op != IQ_OUT_RESIDUAL || a.n == 1) && chain_h_applies(hs.W, a.n, rows);
+            // stages whose K one gemvw workgroup covers (5..16 rows up to 32
+            // groups, 17..32 rows up to 16): one launch with the epilogue in
+            // it (1.5B int4 / int8 chains at 16 sequences 445 / 382 -> 386 /
+            // 288 us, 7B int8 463 -> 362, with its down stage on gemvw's range
+            // sums).  Other narrow stages at 5..16 rows (an odd number of
+            // groups): the input transform into prepared f16 operands, then
+            // gemvh with bias, residual and per-tile sums of squares in its
+            // own epilogue
+            hs.wroute = (a.out_op != IQ_OUT_RESIDUAL || a.n == 1) && chain_w_applies(hs.W, a.n, rows, pair);
+            hs.hroute = !hs.wroute && !pair && (a.out_op != IQ_OUT_RESIDUAL || a.n == 1) && chain_h_applies(hs.W, a.n, rows);
             continue;
         }
         // slices of whole 4-group blocks (measured: fewer, fatter waves beat
@@ -900,7 +907,7 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
         std::vector<int> producer(static_cast<size_t>(n), -1);
         auto ssq_count = [&](int e) {
             const HostStage& hp = prog[size_t(e)];
-            return (hp.fused_r > 1 || hp.hroute) ? int((hp.st.mat[0].N + 15) / 16) : int((hp.epi.ncols + 255) / 256);
+            return (hp.fused_r > 1 || hp.hroute || hp.wroute) ? int((hp.st.mat[0].N + 15) / 16) : int((hp.epi.ncols + 255) / 256);
         };
         for (const auto& l : links)
             if (rows_of(l.second) > 1 && ssq_count(l.first) <= 256) producer[size_t(l.second)] = l.first;
@@ -909,7 +916,7 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
         for (int s = 0; s < n; s++) {
             HostStage& h = prog[size_t(s)];
             if (h.rows == 1) continue;
-            if (h.fused_r == 1)
+            if (h.fused_r == 1 && !h.wroute)
                 part = std::max<int64_t>(part, chain_rows_partials(h.W, h.st.nmat, h.rows, kStreamPartialFloats));
             if (stages[s].in_op != IQ_IN_RMSNORM) continue;
             const int pe = producer[size_t(s)];
@@ -975,13 +982,17 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
 hipError_t chain_run(const Chain* ch, hipStream_t stream) {
     for (const HostStage& h : ch->stages) {
         hipError_t e;
-        if (h.rows > 1 && h.fused_r == 1 && h.hroute) {
+        if (h.rows > 1 && h.fused_r == 1 && (h.hroute || h.wroute)) {
             if (h.own_ssq) {
                 const int K = int(h.W[0].cols);
                 ssq_kernel<<<dim3(unsigned(h.in.ssq_n), unsigned(h.rows)), 256, 0, stream>>>(h.in.x, K, h.in.ssq_n, h.ssq);
             }
-            e = launch_chain_h(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.res, h.epi.ssq_out, ch->hxq,
-                               ch->hxmeta, stream);
+            if (h.wroute)
+                e = launch_chain_w(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.swiglu != 0, h.epi.res,
+                                   h.epi.ssq_out, stream);
+            else
+                e = launch_chain_h(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.res, h.epi.ssq_out, ch->hxq,
+                                   ch->hxmeta, stream);
         } else if (h.rows > 1 && h.fused_r == 1) {
             e = run_rows_stage(h, ch->rpart, ch->rpart_floats, stream);
         } else {

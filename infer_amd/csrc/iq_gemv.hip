@@ -146,8 +146,11 @@ struct GemvParams {
     // gemvh epilogue (chain stages): y = res + (sum + bias) when res, and
     // the sum of squares of each 16-column tile of each output row into
     // ssq_out[m * ntiles + tile] when ssq_out
+    // (gemvw's chain instances the same, and with pair the SwiGLU of the two
+    // matrices, whose 16-row tiles then alternate in the tile order)
     const float* res;
     float* ssq_out;
+    int pair;
 };
 
 // ------------------------------------------------------------------ chain prologue
@@ -2328,10 +2331,10 @@ __global__ __launch_bounds__(512, (PRO && (LOOP || (KIND == 0 && MB == 2))) ? 2 
 // 5..32 rows, each wave keeping its share of the activations in registers:
 // wave w of a workgroup takes NG groups of K (the workgroup's nw waves a
 // range of gs = nw NG groups, at most 32 at up to 16 rows and 16 at 17..32)
-// and walks the workgroup's 16-row tiles over them, its f16 split operands
+// and walks the workgroup's 16-column tiles over them, its f16 split operands
 // made once, in registers (through the wave's own LDS, no barrier), and the
 // next D tiles' weights, scales and zero points in flight; the waves' sums
-// of CH tiles are added from LDS in wave order.  One workgroup of up to 8
+// of CH tiles are added from LDS.  One workgroup of up to 8
 // waves per CU, the tiles dealt out evenly, so the weights stream from the
 // first to the last instruction; rows of up to 32 (16) groups need no range
 // sums and no reduction launch, and no call needs a preparation launch.
@@ -2362,7 +2365,11 @@ struct GwShape {
     static constexpr int WAVEB = (OPB > PARTB ? OPB : PARTB) + FACB;
 };
 
-template <int KIND, int MB2, int NG>
+// PRO (chain stages): activations through the prologue's gather and RMSNorm
+// (pro_x_offset, pro_norm8; the row factors, in ProScale's order, multiply
+// the group factors), outputs through the stage's epilogue, or with to_part
+// as range sums.
+template <int KIND, int MB2, int NG, bool PRO>
 __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
     using S = GwShape<KIND, MB2, NG>;
     constexpr bool PK = MB2 == 1;
@@ -2375,19 +2382,55 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
     const int g0 = range * p.gs + wave * NG;
     const int gend = range * p.gs + p.gs < G ? range * p.gs + p.gs : G;
     const int ng = gend - g0 < 0 ? 0 : (gend - g0 < NG ? gend - g0 : NG);
-    const int t0 = int(int64_t(rb) * p.ntiles / p.nrb), t1 = int(int64_t(rb + 1) * p.ntiles / p.nrb);
+    // (a SwiGLU pair's tiles stay together)
+    const int unit = PRO && p.pair ? 2 : 1, units = p.ntiles / unit;
+    const int t0 = unit * int(int64_t(rb) * units / p.nrb), t1 = unit * int(int64_t(rb + 1) * units / p.nrb);
+    auto select = [&](int tile) {
+        if (PRO && p.pair) return TileSel{p.mat[tile & 1], int64_t(tile >> 1) * 16};
+        return select_tile(p, tile);
+    };
     const int row_bytes = int(KIND == 1 ? p.K / 2 : p.K);
     int8_t* const mine = wlds + wave * S::WAVEB;
 
-    // 1. this wave's activations: its groups of every row
+    // 1. with RMSNorm, the partial sums of squares of this thread's row(s):
+    //    16 lanes a row, a row per 16 threads now (any others later); then
+    //    this wave's activations: its groups of every row
+    __shared__ float rsc[PRO ? kMaxRowsGemv : 1];
+    const int rstep = int(blockDim.x) >> 4;
+    float sq[PRO ? 16 : 1];
+    auto request_ssq = [&](int m, float (&v)[PRO ? 16 : 1]) {
+        const rsrc_t r = make_rsrc(p.ssq, p.norm ? int64_t(p.M) * p.ssq_n * 4 : 0);
+#pragma unroll
+        for (int k = 0; k < (PRO ? 16 : 0); k++) {
+            const int b = ln + 16 * k;
+            v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                 r, (m < p.M && b < p.ssq_n) ? uint32_t(m * p.ssq_n + b) * 4 : kOob, 0, 0));
+        }
+    };
+    auto finish_ssq = [&](int m, const float (&v)[PRO ? 16 : 1]) {
+        double part = 0.0, ss = 0.0;
+#pragma unroll
+        for (int k = 0; k < (PRO ? 16 : 0); k++) part += double(v[k]);
+#pragma unroll
+        for (int j = 0; j < 16; j++) ss += __shfl(part, j, 16);
+        if (ln == 0 && m < p.M) rsc[m] = 1.0f / __builtin_sqrtf(float(ss / double(p.K)) + p.eps);
+    };
+    if constexpr (PRO) request_ssq(tid >> 4, sq);
     float xv[S::NX][8];
+    uint4 nwv[PRO ? NG : 1];
     {
-        const rsrc_t rxx = make_rsrc(p.x, int64_t(p.M) * p.K * 4);
+        const rsrc_t rxx = make_rsrc(p.x, int64_t(p.M) * (PRO ? p.xstride : p.K) * 4);
+        const rsrc_t rn = make_rsrc(PRO ? p.norm : nullptr, PRO && p.norm ? p.K * 2 : 0);
+#pragma unroll
+        for (int i = 0; i < (PRO ? NG : 0); i++)
+            nwv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   rn, i < ng ? uint32_t((g0 + i) * kGroup + ln * 8) * 2 : kOob, 0, 0));
 #pragma unroll
         for (int u = 0; u < S::NX; u++) {
             const int t = lane + 64 * u, pr = t >> 4;
             const int m = pr % S::ROWS, i = pr / S::ROWS;
-            const uint32_t o = (i < ng && m < p.M) ? uint32_t((int64_t(m) * p.K + int64_t(g0 + i) * kGroup + ln * 8) * 4) : kOob;
+            const int64_t col = int64_t(g0 + i) * kGroup + ln * 8;
+            const uint32_t o = (i < ng && m < p.M) ? (PRO ? pro_x_offset(p, m, col) : uint32_t((int64_t(m) * p.K + col) * 4)) : kOob;
             const float4_t a = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rxx, o, 0, 0));
             const float4_t b = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rxx, o, 16, 0));
 #pragma unroll
@@ -2406,7 +2449,7 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
     Buf bufs[S::D];
     auto request = [&](Buf& b, int tile) {
         const bool ok = tile < t1;
-        const TileSel ts = select_tile(p, ok ? tile : t0);
+        const TileSel ts = select(ok ? tile : t0);
         const int64_t left = ts.m.N - ts.row0;
         const int64_t rows = ok ? (left < 16 ? left : 16) : 0;
         const rsrc_t rq = make_rsrc_wave(ts.m.q + ts.row0 * row_bytes, rows * row_bytes);
@@ -2433,8 +2476,12 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
                                                            rq, vq + o, (g0 + i) * (KIND == 1 ? 64 : 128) + h * 16, 0));
         }
     };
+    // (the instance whose registers the operands, the prologue and int8
+    // weights would overfill requests its second tile after the conversion)
+    constexpr bool TIGHT = PRO && KIND == 0 && MB2 == 2 && NG == 4;
+    constexpr int EARLY = TIGHT ? 1 : S::D;
 #pragma unroll
-    for (int d = 0; d < S::D; d++) request(bufs[d], t0 + d);
+    for (int d = 0; d < EARLY; d++) request(bufs[d], t0 + d);
     // 3. the operands, group by group through the wave's own LDS
     half8_t ops[NG][S::BLK][S::OPS];
 #pragma unroll
@@ -2449,6 +2496,9 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
                 const int m = (lane >> 4) + 4 * u;  // row in the block
                 half8_t ho, lo;
                 float fac;
+                if constexpr (PRO) {
+                    if (p.norm) pro_norm8(xv[(i * S::BLK + b) * TB + u], nwv[i]);
+                }
                 xh_split8<KIND == 1>(xv[(i * S::BLK + b) * TB + u], ho, lo, fac);
                 const int qq = ln >> 2, jj = ln & 3;
                 if (PK) {
@@ -2464,6 +2514,22 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
 #pragma unroll
             for (int o = 0; o < S::OPS; o++) ops[i][b][o] = dst[o * S::CS + lane];
             __builtin_amdgcn_wave_barrier();
+        }
+    }
+#pragma unroll
+    for (int d = EARLY; d < S::D; d++) request(bufs[d], t0 + d);
+    if constexpr (PRO) {
+        if (p.norm) {  // uniform
+            finish_ssq(tid >> 4, sq);
+            for (int m = (tid >> 4) + rstep; m - (tid >> 4) < p.M; m += rstep) {
+                float v[16];
+                request_ssq(m, v);
+                finish_ssq(m, v);
+            }
+            __syncthreads();
+            float* fs = reinterpret_cast<float*>(mine + S::WAVEB - S::FACB);
+            const int m = (lane >> 4) % S::BLK * 16 + ln;  // factor `lane` = (group, block, row)
+            if (lane < NG * S::BLK * 16 && m < S::ROWS) fs[lane] *= rsc[m < p.M ? m : 0];
         }
     }
     // 4. the tiles
@@ -2519,26 +2585,68 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
 #pragma unroll
         for (int b = 0; b < S::BLK; b++) slot[b * 64 + lane] = acc[b];
     };
-    // the waves' sums of tiles [c, c + n), in wave order
-    auto finish = [&](int c, int n, int odd) {
-        for (int it = wave; it < n * S::BLK; it += nw) {
-            const int b = it % S::BLK, tile = c + it / S::BLK;
-            const float4_t* src = reinterpret_cast<const float4_t*>(wlds) + odd * (S::CH * 64 * S::BLK) + it * 64 + lane;
-            float4_t sum = src[0];
+    // a tile's sums over the waves, the even and the odd ones apart (in wave
+    // order where the registers are full) (lane: rows 4q .. 4q + 3 of the
+    // block, column ln)
+    auto total = [&](int odd, int item) {
+        const float4_t* src = reinterpret_cast<const float4_t*>(wlds) + odd * (S::CH * 64 * S::BLK) + item * 64 + lane;
+        float4_t sum = src[0], other = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (TIGHT) {
             for (int w = 1; w < nw; w++) sum += src[w * (S::WAVEB / 16)];
-            if (PK) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) sum[r] += __shfl_down(sum[r], 32, 64);
+        } else {
+            for (int w = 1; w < nw; w += 2) {
+                other += src[w * (S::WAVEB / 16)];
+                if (w + 1 < nw) sum += src[(w + 1) * (S::WAVEB / 16)];
             }
-            const TileSel ts = select_tile(p, tile);
+            sum += other;
+        }
+        if (PK) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[r] += __shfl_down(sum[r], 32, 64);
+        }
+        return sum;
+    };
+    // the outputs of tiles [c, c + n)
+    auto finish = [&](int c, int n, int odd) {
+        for (int it = wave; it < n / unit * S::BLK; it += nw) {
+            const int b = it % S::BLK, first = it / S::BLK * unit, tile = c + first;
+            float4_t sum = total(odd, first * S::BLK + b);
+            const TileSel ts = select(tile);
             const int64_t row = ts.row0 + ln;
-            if (row >= ts.m.N || (PK && q >= 2)) continue;
+            const bool ok = row < ts.m.N && !(PK && q >= 2);
+            const bool to_part = PRO ? p.to_part != 0 : p.S > 1;
+            const float bias = !to_part && ok && ts.m.bias ? bf16_to_f32(ts.m.bias[row]) : 0.0f;
+            if (PRO && p.pair) {
+                // silu(g) * u  (kernels/ops/elementwise.cu:6-11)
+                const float4_t up = total(odd, (first + 1) * S::BLK + b);
+                const float bu = ok && p.mat[1].bias ? bf16_to_f32(p.mat[1].bias[row]) : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float g = sum[r] + bias;
+                    sum[r] = g / (1.0f + expf(-g)) * (up[r] + bu);
+                }
+            }
+            float sqr[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int m = 16 * b + 4 * q + r;
-                if (m >= p.M) continue;
-                if (p.S == 1) ts.m.y[int64_t(m) * ts.m.N + row] = sum[r] + (ts.m.bias ? bf16_to_f32(ts.m.bias[row]) : 0.0f);
-                else p.part[(int64_t(range) * p.M + m) * (int64_t(p.ntiles) * 16) + int64_t(tile) * 16 + ln] = sum[r];
+                if (!ok || m >= p.M) continue;
+                if (to_part) {
+                    p.part[(int64_t(range) * p.M + m) * (int64_t(p.ntiles) * 16) + int64_t(tile) * 16 + ln] = sum[r];
+                    continue;
+                }
+                float v = PRO && p.pair ? sum[r] : sum[r] + bias;
+                if (PRO && p.res) v = p.res[int64_t(m) * ts.m.N + row] + v;
+                ts.m.y[int64_t(m) * ts.m.N + row] = v;
+                sqr[r] = v * v;
+            }
+            if (PRO && p.ssq_out) {  // (one matrix, or a pair: its tiles)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = 16 * b + 4 * q + r;
+                    const float sum16 = row16_sumf(sqr[r]);
+                    if (ln == 0 && m < p.M && !(PK && q >= 2)) p.ssq_out[m * units + tile / unit] = sum16;
+                }
             }
         }
     };
@@ -2565,11 +2673,55 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
     finish(c, t1 - c, odd);
 }
 
-template <int KIND, int MB2, int NG>
+template <int KIND, int MB2, int NG, bool PRO>
 void launch_gemvw_t(const GemvParams& p, unsigned grid, int nw, hipStream_t stream) {
     const size_t lds = size_t(nw) * GwShape<KIND, MB2, NG>::WAVEB;
-    allow_big_lds<gemvw_kernel<KIND, MB2, NG>>();
-    gemvw_kernel<KIND, MB2, NG><<<grid, unsigned(64 * nw), lds, stream>>>(p);
+    allow_big_lds<gemvw_kernel<KIND, MB2, NG, PRO>>();
+    gemvw_kernel<KIND, MB2, NG, PRO><<<grid, unsigned(64 * nw), lds, stream>>>(p);
+}
+
+template <int KIND, bool PRO>
+void launch_gemvw_k(const GemvParams& p, int ng, unsigned grid, int nw, hipStream_t stream) {
+    if (p.M > 16) {
+        launch_gemvw_t<KIND, 4, 2, PRO>(p, grid, nw, stream);
+    } else if (p.M > 8) {
+        if (ng == 4) launch_gemvw_t<KIND, 2, 4, PRO>(p, grid, nw, stream);
+        else launch_gemvw_t<KIND, 2, 2, PRO>(p, grid, nw, stream);
+    } else {
+        if (ng == 4) launch_gemvw_t<KIND, 1, 4, PRO>(p, grid, nw, stream);
+        else launch_gemvw_t<KIND, 1, 2, PRO>(p, grid, nw, stream);
+    }
+}
+
+// gemvw's ranges and workgroups for M rows, `units` 16-row tiles (or SwiGLU
+// pairs of them): S ranges of gs groups, nw waves of ng groups a workgroup,
+// nrb workgroups a range.  ok: G is whole sets of ng groups.
+struct GwPlan {
+    int ng = 0, S = 0, gs = 0, nw = 0, nrb = 0;
+    bool ok = false;
+};
+
+GwPlan gemvw_plan(int64_t G, int M, int units) {
+    GwPlan pl;
+    // groups a wave: 4 (2 from 17 rows: their operands fill the registers),
+    // or 2 where G leaves a remainder and on short rows, whose few waves
+    // would otherwise leave half the CU's registers unused (1.5B gate|up, G =
+    // 12, at 16 rows int4 / int8 14.0 / 15.0 -> 10.9 / 11.6 us, 5 rows 10.7
+    // / 12.1 -> 10.3 / 10.2); whole sets only
+    pl.ng = M <= 16 && G % 4 == 0 && G > 16 ? 4 : 2;
+    if (M < 5 || M > kMaxRowsGemv || G % pl.ng) return pl;
+    pl.S = int((G + 8 * pl.ng - 1) / (8 * pl.ng));
+    pl.gs = int((G + pl.S - 1) / pl.S);
+    pl.gs = (pl.gs + pl.ng - 1) / pl.ng * pl.ng;
+    pl.S = int((G + pl.gs - 1) / pl.gs);
+    pl.nw = pl.gs / pl.ng;
+    const int slots = device_cu_count() * (8 / pl.nw);
+    pl.nrb = std::min(units, std::max(1, slots / pl.S));
+    // (one or two tiles a workgroup: two each, so that no CU waits for a
+    // second workgroup)
+    if (units < 2 * pl.nrb && units > pl.nrb) pl.nrb = (units + 1) / 2;
+    pl.ok = true;
+    return pl;
 }
 
 // gemvw or the other kernels (both measured in a graph, us, others -> gemvw):
@@ -2593,60 +2745,29 @@ bool gemvw_preferred(int M, int tiles, int64_t K, int kind) {
 // groups, or the partial sums would not fit).
 bool launch_gemvw(const float* x, const QView* W, const uint16_t* const* bias, float* const* y, int n, int M, Workspace* ws,
                   hipStream_t stream, hipError_t* err) {
-    const int64_t K = W[0].cols, G = W[0].groups;
     GemvParams p{};
     int tiles = 0;
     for (int i = 0; i < n; i++) {
         p.mat[i] = MatRef{W[i].q, W[i].scales, W[i].zeros, bias[i], y[i], W[i].rows, tiles};
         tiles += int((W[i].rows + 15) / 16);
     }
-    // groups a wave: 4 (2 from 17 rows: their operands fill the registers),
-    // or 2 where G leaves a remainder; whole sets only
-    const int ng = M <= 16 && G % 4 == 0 ? 4 : 2;
-    if (G % ng) return false;
-    int S = int((G + 8 * ng - 1) / (8 * ng));
-    int gs = int((G + S - 1) / S);
-    gs = (gs + ng - 1) / ng * ng;
-    S = int((G + gs - 1) / gs);
-    const int nw = gs / ng;
-    if (S > 1 && int64_t(S) * M * tiles * 16 > ws->part_floats) return false;
-    const int slots = device_cu_count() * (8 / nw);
+    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles);
+    if (!pl.ok || (pl.S > 1 && int64_t(pl.S) * M * tiles * 16 > ws->part_floats)) return false;
     p.nmat = n;
-    p.K = K;
-    p.G = G;
+    p.K = W[0].cols;
+    p.G = W[0].groups;
     p.x = x;
     p.M = M;
-    p.gs = gs;
-    p.S = S;
+    p.gs = pl.gs;
+    p.S = pl.S;
+    p.nrb = pl.nrb;
     p.ntiles = tiles;
-    p.nrb = std::min(tiles, std::max(1, slots / S));
-    if (tiles < 2 * p.nrb && tiles > p.nrb) p.nrb = (tiles + 1) / 2;
     p.part = ws->partials;
-    const unsigned grid = unsigned(p.nrb * S);
-    const bool i4 = W[0].kind == 1;
-    if (M > 16) {
-        if (i4) launch_gemvw_t<1, 4, 2>(p, grid, nw, stream);
-        else launch_gemvw_t<0, 4, 2>(p, grid, nw, stream);
-    } else if (M > 8) {
-        if (ng == 4) {
-            if (i4) launch_gemvw_t<1, 2, 4>(p, grid, nw, stream);
-            else launch_gemvw_t<0, 2, 4>(p, grid, nw, stream);
-        } else {
-            if (i4) launch_gemvw_t<1, 2, 2>(p, grid, nw, stream);
-            else launch_gemvw_t<0, 2, 2>(p, grid, nw, stream);
-        }
-    } else {
-        if (ng == 4) {
-            if (i4) launch_gemvw_t<1, 1, 4>(p, grid, nw, stream);
-            else launch_gemvw_t<0, 1, 4>(p, grid, nw, stream);
-        } else {
-            if (i4) launch_gemvw_t<1, 1, 2>(p, grid, nw, stream);
-            else launch_gemvw_t<0, 1, 2>(p, grid, nw, stream);
-        }
-    }
+    const unsigned grid = unsigned(pl.nrb * pl.S);
+    if (W[0].kind == 1) launch_gemvw_k<1, false>(p, pl.ng, grid, pl.nw, stream);
+    else launch_gemvw_k<0, false>(p, pl.ng, grid, pl.nw, stream);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && S > 1) {
-        const int64_t outs = int64_t(M) * tiles * 16;
+    if (e == hipSuccess && pl.S > 1) {
         launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
@@ -3155,6 +3276,7 @@ namespace {
 struct RowsSetup {
     GemvParams p{};
     bool q = false;  // gemvq (else gemvr)
+    GwPlan w;        // gemvw, when ok
     int S = 0;
     unsigned grid = 0;
     bool ok = false;
@@ -3177,6 +3299,17 @@ RowsSetup rows_setup(const QView* W, int n, int M, int64_t part_floats) {
     r.p.ntiles = tiles;
     r.p.to_part = 1;
     const int cus = device_cu_count();
+    r.w = gemvw_plan(G, M, tiles);
+    if (r.w.ok && int64_t(r.w.S) * M * tiles * 16 <= part_floats) {
+        r.p.gs = r.w.gs;
+        r.p.S = r.w.S;
+        r.p.nrb = r.w.nrb;
+        r.S = r.w.S;
+        r.grid = unsigned(r.w.nrb * r.w.S);
+        r.ok = true;
+        return r;
+    }
+    r.w.ok = false;
     const bool use_q = M >= 17 || (M >= 9 && W[0].kind == 1 && tiles >= 1024);
     if (!use_q) {
         // launch_gemvr's ranges
@@ -3249,7 +3382,10 @@ hipError_t launch_chain_rows(const QView* W, int n, int M, const RowsIn& in, flo
     p.part = part;
     *S = r.S;
     const int kind = W[0].kind;
-    if (!r.q) {
+    if (r.w.ok) {
+        if (kind == 1) launch_gemvw_k<1, true>(p, r.w.ng, r.grid, r.w.nw, stream);
+        else launch_gemvw_k<0, true>(p, r.w.ng, r.grid, r.w.nw, stream);
+    } else if (!r.q) {
         if (M <= 8) {
             if (kind == 1) gemvr_kernel<1, true, 8, true><<<r.grid, 512, 0, stream>>>(p);
             else gemvr_kernel<0, true, 8, true><<<r.grid, 512, 0, stream>>>(p);
@@ -3274,6 +3410,46 @@ hipError_t launch_chain_rows(const QView* W, int n, int M, const RowsIn& in, flo
             else gemvq_kernel<0, 4, 2, false, true><<<r.grid, 512, 0, stream>>>(p);
         }
     }
+    return hipGetLastError();
+}
+
+bool chain_w_applies(const QView* W, int n, int M, bool pair) {
+    const int tiles = pair ? int((W[0].rows + 15) / 16) : total_tiles(W, n);
+    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles);
+    return pl.ok && pl.S == 1;
+}
+
+hipError_t launch_chain_w(const QView* W, int n, int M, const RowsIn& in, const uint16_t* const* bias, float* const* y,
+                          bool pair, const float* res, float* ssq_out, hipStream_t stream) {
+    GemvParams p{};
+    int tiles = 0;
+    for (int i = 0; i < n; i++) {
+        p.mat[i] = MatRef{W[i].q, W[i].scales, W[i].zeros, bias[i], pair ? y[0] : y[i], W[i].rows, tiles};
+        tiles += int((W[i].rows + 15) / 16);
+    }
+    const GwPlan pl = gemvw_plan(W[0].groups, M, pair ? tiles / 2 : tiles);
+    if (!pl.ok || pl.S != 1) return hipErrorInvalidValue;
+    p.nmat = n;
+    p.K = W[0].cols;
+    p.G = W[0].groups;
+    p.M = M;
+    p.gs = pl.gs;
+    p.S = 1;
+    p.nrb = pl.nrb;
+    p.ntiles = tiles;
+    p.x = in.x;
+    p.xstride = in.xstride;
+    p.gqa_hd = in.gqa_hd;
+    p.gqa_span = in.gqa_span;
+    p.norm = in.norm;
+    p.ssq = in.ssq;
+    p.ssq_n = in.ssq_n;
+    p.eps = in.eps;
+    p.res = res;
+    p.ssq_out = ssq_out;
+    p.pair = pair ? 1 : 0;
+    if (W[0].kind == 1) launch_gemvw_k<1, true>(p, pl.ng, unsigned(pl.nrb), pl.nw, stream);
+    else launch_gemvw_k<0, true>(p, pl.ng, unsigned(pl.nrb), pl.nw, stream);
     return hipGetLastError();
 }
 

@@ -135,6 +135,15 @@ hipError_t launch_chain_h(const QView* W, int n, int M, const RowsIn& in, const 
                           float* const* y, const float* res, float* ssq_out, int8_t* xq, float* xmeta,
                           hipStream_t stream);
 
+// A chain stage at 5..32 rows whose K one gemvw workgroup covers (at most 32
+// groups, 16 from 17 rows on): one launch, input transform, GEMV and epilogue
+// (y = (res +) sum + bias, or with pair silu(gate) * up), and when ssq_out
+// the sum of squares of each 16-column tile of each output row
+// (ssq_out[m * tiles + tile]).
+bool chain_w_applies(const QView* W, int n, int M, bool pair);
+hipError_t launch_chain_w(const QView* W, int n, int M, const RowsIn& in, const uint16_t* const* bias, float* const* y,
+                          bool pair, const float* res, float* ssq_out, hipStream_t stream);
+
 // A validated stage program on the device (iq_chain.hip).
 struct Chain;
 void chain_destroy(Chain* ch);

@@ -61,6 +61,13 @@ __device__ __forceinline__ float row16_max(float v) {
     v = fmaxf(v, __int_as_float(row_ror<1>(__float_as_int(v))));
     return v;
 }
+__device__ __forceinline__ float row16_sumf(float v) {
+    v += __int_as_float(row_ror<8>(__float_as_int(v)));
+    v += __int_as_float(row_ror<4>(__float_as_int(v)));
+    v += __int_as_float(row_ror<2>(__float_as_int(v)));
+    v += __int_as_float(row_ror<1>(__float_as_int(v)));
+    return v;
+}
 __device__ __forceinline__ int row16_and(int v) {
     v &= row_ror<8>(v);
     v &= row_ror<4>(v);
