@@ -1,11 +1,9 @@
 // iq_quant.hip -- on-device quantize + pack and the quantised embedding
 // gather for gfx950.
 //
-// quantize: bit-exact to llm::quantize (src/quant.cpp:34-84).  Whole-group
-// rows (cols % 128 == 0, quantize8_kernel): one wave64 covers eight
-// 128-column groups of one row, 8 lanes per group, each lane 16 consecutive
-// columns (two 16-byte loads of bf16).  Ragged rows (quantize_kernel): four
-// groups per wave, each 16-lane DPP row one group, 8 columns per lane.
+// quantize: bit-exact to llm::quantize (src/quant.cpp:34-84): one wave64
+// covers eight 128-column groups of one row, 8 lanes per group, each lane 16
+// consecutive columns (two 16-byte loads of bf16).
 // The group's absmax (int8) or [min,max] widened to 0 (int4) is reduced
 // inside the group's lanes; every lane then derives the same bf16 scale and
 // writes its codes, so stores stay coalesced.  Groups whose scale is
@@ -29,27 +27,6 @@ namespace iq {
 namespace {
 
 constexpr int kQThreads = 256;
-
-// Max / min over the 16 lanes of a DPP row (one quantisation group), by
-// row rotations: exact in any order.  v_max_f32 / v_min_f32 return the other
-// operand for a NaN (IEEE maxNum), which is what the reference's `a < b`
-// updates do; the running values start at 0 and never become NaN.
-template <int N>
-__device__ __forceinline__ float row_ror_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float row16_maxf(float v) {
-    v = __builtin_fmaxf(v, row_ror_f<8>(v));
-    v = __builtin_fmaxf(v, row_ror_f<4>(v));
-    v = __builtin_fmaxf(v, row_ror_f<2>(v));
-    return __builtin_fmaxf(v, row_ror_f<1>(v));
-}
-__device__ __forceinline__ float row16_minf(float v) {
-    v = __builtin_fminf(v, row_ror_f<8>(v));
-    v = __builtin_fminf(v, row_ror_f<4>(v));
-    v = __builtin_fminf(v, row_ror_f<2>(v));
-    return __builtin_fminf(v, row_ror_f<1>(v));
-}
 
 // Reference clamp (std::max(lo, std::min(hi, v))).
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -112,172 +89,6 @@ __device__ __forceinline__ QScale qscale(float s) {
     return q;
 }
 
-template <int KIND, bool FAST>
-__global__ __launch_bounds__(kQThreads) void quantize_kernel(const uint16_t* __restrict__ w,
-                                                             int64_t rows, int64_t cols, int64_t G,
-                                                             int64_t quads, uint8_t* __restrict__ q,
-                                                             uint16_t* __restrict__ scales,
-                                                             uint8_t* __restrict__ zeros) {
-    const int lane = threadIdx.x & 63;
-    // Grid-stride over (row, 4-group quad) items; the bf16 values of the
-    // next QD items are requested before the current one is converted.
-    // (row, quad) cursors advance without division (a 64-bit division is a
-    // long instruction sequence on the GPU).
-    const int64_t items = rows * quads;
-    const int64_t stride = int64_t(gridDim.x) * (kQThreads / 64);
-    const int64_t first = int64_t(blockIdx.x) * (kQThreads / 64) + (threadIdx.x >> 6);
-    if (first >= items) return;
-    const int64_t sr = stride / quads, sq = stride % quads;
-    struct Cursor {
-        int64_t r, qd;
-    };
-    auto advance = [&](Cursor& c) {
-        c.r += sr;
-        c.qd += sq;
-        if (c.qd >= quads) {
-            c.qd -= quads;
-            c.r += 1;
-        }
-    };
-    // Unconditional buffer loads (a row past the end or a group past the
-    // row reads zero without a memory access): no branch around the load,
-    // so the wait before an item's use covers only that item's request.
-    auto fetch = [&](const Cursor& c) {
-        if (!FAST) return make_uint4(0, 0, 0, 0);
-        // (the cursor is the same in every lane of the wave)
-        const int64_t r = (int64_t(__builtin_amdgcn_readfirstlane(uint32_t(c.r >> 32))) << 32) |
-                          int64_t(__builtin_amdgcn_readfirstlane(uint32_t(c.r)));
-        const bool rok = r < rows;
-        const rsrc_t rw = make_rsrc(w + (rok ? r : 0) * cols, rok ? cols * 2 : 0);
-        const int64_t gg = c.qd * 4 + (lane >> 4);
-        const uint32_t off = gg < G ? uint32_t((gg * kGroup + (lane & 15) * 8) * 2) : kOob;
-        return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
-    };
-    constexpr int QD = 2;
-    Cursor cc{first / quads, first % quads}, fc = cc;
-    uint4 ring[QD];
-#pragma unroll
-    for (int d = 0; d < QD; d++) {
-        ring[d] = fetch(fc);
-        advance(fc);
-    }
-    for (; cc.r < rows; advance(cc)) {
-    const uint4 cur = ring[0];
-#pragma unroll
-    for (int d = 0; d < QD - 1; d++) ring[d] = ring[d + 1];
-    ring[QD - 1] = fetch(fc);
-    advance(fc);
-    const int64_t r = cc.r;
-    const int64_t g = cc.qd * 4 + (lane >> 4);  // this 16-lane row's group
-    const bool gvalid = g < G;
-    const int64_t c0 = g * kGroup + (lane & 15) * 8;    // first of my 8 columns
-    const uint16_t* wr = w + r * cols;
-
-    float v[8];
-    if (FAST) {  // cols % 128 == 0: whole groups, 16-byte aligned rows
-        const uint4 raw = cur;
-        const uint32_t wd[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[2 * i] = __uint_as_float(wd[i] << 16);
-            v[2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = (gvalid && c0 + i < cols) ? bf16_to_f32(wr[c0 + i]) : 0.0f;
-    }
-    const int nvalid = FAST ? 8 : (gvalid ? int(cols - c0 < 0 ? 0 : (cols - c0 < 8 ? cols - c0 : 8)) : 0);
-
-    if (KIND == 0) {
-        // amax = std::max(amax, fabs(v)) in column order; comparisons skip NaN.
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float a = __builtin_fabsf(v[i]);
-            if (i < nvalid && amax < a) amax = a;
-        }
-        amax = row16_maxf(amax);
-        const uint16_t sb = f32_to_bf16(amax > 0.0f ? amax / 127.0f : 1.0f);
-        const QScale qs = qscale(bf16_to_f32(sb));
-        uint32_t lo = 0, hi = 0;
-        // every group of the wave on the fast path (the usual case), or the
-        // general one (non-finite values, tiny scales) for the whole wave
-        const bool plain = qs.up == 1.0f && qs.s < 3.0e38f;
-        if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
-            const float rf = __builtin_amdgcn_rcpf(qs.s);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int c = clampi(qdiv_fast(v[i], qs.s, rf), -127, 127);
-                const uint32_t b = uint32_t(uint8_t(int8_t(c)));
-                if (i < 4) lo |= b << (8 * i);
-                else hi |= b << (8 * (i - 4));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int c = clampi(qdiv(v[i] * qs.up, qs.s, qs.r()), -127, 127);
-                const uint32_t b = uint32_t(uint8_t(int8_t(c)));
-                if (i < 4) lo |= b << (8 * i);
-                else hi |= b << (8 * (i - 4));
-            }
-        }
-        if (!gvalid) continue;
-        if ((lane & 15) == 0) scales[r * G + g] = sb;
-        uint8_t* qr = q + r * cols + c0;
-        if (FAST) {
-            *reinterpret_cast<uint2*>(qr) = make_uint2(lo, hi);
-        } else {
-            for (int i = 0; i < nvalid; i++) qr[i] = uint8_t((i < 4 ? lo >> (8 * i) : hi >> (8 * (i - 4))) & 0xFF);
-        }
-    } else {
-        // lo = std::min(lo, v), hi = std::max(hi, v), both starting at 0.
-        float mn = 0.0f, mx = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (i < nvalid) {
-                if (v[i] < mn) mn = v[i];
-                if (mx < v[i]) mx = v[i];
-            }
-        }
-        mn = row16_minf(mn);
-        mx = row16_maxf(mx);
-        const uint16_t sb = f32_to_bf16(mx > mn ? (mx - mn) / 15.0f : 1.0f);
-        const QScale qs = qscale(bf16_to_f32(sb));
-        uint32_t packed = 0;
-        int z;
-        const bool plain = qs.up == 1.0f && qs.s < 3.0e38f;
-        if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
-            const float rf = __builtin_amdgcn_rcpf(qs.s);
-            z = clampi(qdiv_fast(-mn, qs.s, rf), 0, 15);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int c = clampi(qdiv_fast(v[i], qs.s, rf) + z, 0, 15);
-                packed |= uint32_t(c) << (4 * i);
-            }
-        } else {
-            z = clampi(qdiv(-mn * qs.up, qs.s, qs.r()), 0, 15);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int c = clampi(qdiv(v[i] * qs.up, qs.s, qs.r()) + z, 0, 15);
-                packed |= uint32_t(c) << (4 * i);
-            }
-        }
-        if (!gvalid) continue;
-        if ((lane & 15) == 0) {
-            scales[r * G + g] = sb;
-            zeros[r * G + g] = uint8_t(z);
-        }
-        // (r*cols + c0) is even: the lane owns whole bytes.
-        uint8_t* qb = q + (r * cols + c0) / 2;
-        if (FAST) {
-            *reinterpret_cast<uint32_t*>(qb) = packed;
-        } else {
-            for (int i = 0; i < nvalid; i += 2) qb[i / 2] = uint8_t((packed >> (4 * i)) & 0xFF);
-        }
-    }
-    }
-}
-
 // Max / min over the 8 lanes of a half DPP row (one quantisation group of
 // quantize8_kernel): half-row mirror, then two quad permutations.
 template <int CTRL>
@@ -332,10 +143,9 @@ __device__ __forceinline__ uint32_t pack4_b0(int c0, int c1, int c2, int c3) {
     return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
-// quantize for cols % 128 == 0: the arithmetic of quantize_kernel with 8
-// lanes per group and 16 columns per lane (two 16-byte loads), so the
-// per-group work (reductions, the scale's two divisions and its bf16
-// rounding, addresses) is spread over twice the values.  Items are (row,
+// The quantiser: 8 lanes per group and 16 columns per lane (two 16-byte
+// loads), so the per-group work (reductions, the scale's two divisions and
+// its bf16 rounding, addresses) is spread over many values.  Items are (row,
 // 8 groups); rows whose group count is not a multiple of 8 leave the
 // surplus lanes of their last item idle.  A wave walks its items in grid
 // strides with three register sets: the values of the next two items are
@@ -345,7 +155,13 @@ __device__ __forceinline__ uint32_t pack4_b0(int c0, int c1, int c2, int c3) {
 // magnitudes of groups without NaN are compared as unsigned bf16 bits
 // (packed 16-bit maxima), the int4 range with fp32 min / max; a wave
 // holding a NaN takes the reference's comparison loop.
-template <int KIND>
+// RAGGED (cols % 128 != 0): the same requests and stores at any byte offset;
+// columns past the row's end (the next row's values) count as zero, which
+// no group statistic sees, and the lane they begin in stores its codes one
+// byte at a time.  Bound by HBM like the whole-group form (element by
+// element loads and byte stores in all lanes: 15872 x 2146 int4 52.5 ->
+// 28.0 us, 15872 x 2147 int8 56.5 -> 26.9).
+template <int KIND, bool RAGGED>
 __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __restrict__ w, int64_t rows,
                                                               int64_t cols, int64_t G, int64_t octs,
                                                               uint8_t* __restrict__ q, uint16_t* __restrict__ scales,
@@ -374,9 +190,15 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
     };
     auto fetch = [&](const Cursor& c) {
         const bool rok = c.r < rows;
-        const rsrc_t rw = make_rsrc(w + (rok ? c.r : 0) * cols, rok ? cols * 2 : 0);
+        // RAGGED: a resource over the item's columns, whose last chunk runs
+        // into the next row; lane l's 16 columns at 32 l
+        const int64_t r = rok ? c.r : 0, col0 = c.o * (8 * kGroup);
+        const int64_t avail = RAGGED ? std::min<int64_t>(rows * cols - r * cols - col0, 8 * kGroup + 16) : cols;
+        const rsrc_t rw = make_rsrc(w + r * cols + (RAGGED ? col0 : 0), rok ? avail * 2 : 0);
         const int64_t g = c.o * 8 + (lane >> 3);
-        const uint32_t off = g < G ? uint32_t((g * kGroup + sub * 16) * 2) : kOob;
+        uint32_t off;
+        if (RAGGED) off = col0 + lane * 16 < cols ? uint32_t(lane * 32) : kOob;
+        else off = g < G ? uint32_t((g * kGroup + sub * 16) * 2) : kOob;
         Raw x;
         x.a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
         x.b = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 16, 0));
@@ -386,14 +208,27 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
         const int64_t r = cc.r;
         const int64_t g = cc.o * 8 + (lane >> 3);
         const bool gvalid = g < G;
-        const uint32_t wd[8] = {cur.a.x, cur.a.y, cur.a.z, cur.a.w, cur.b.x, cur.b.y, cur.b.z, cur.b.w};
+        uint32_t wd[8] = {cur.a.x, cur.a.y, cur.a.z, cur.a.w, cur.b.x, cur.b.y, cur.b.z, cur.b.w};
+        const int64_t c0 = g * kGroup + sub * 16;
+        const int64_t left = cols - c0;  // columns of the row from this lane's first on
+        const bool edge = RAGGED && (cc.o + 1) * 8 * kGroup > cols;  // wave-uniform: the row ends here
+        if (edge) {
+            if (r + 1 == rows && (cols & 1)) {
+                // the matrix ends inside a 4-byte word, which the buffer
+                // resource cuts off whole: its last value on its own
+                const uint32_t e = w[r * cols + cols - 1];
+#pragma unroll
+                for (int i = 0; i < 8; i++) wd[i] = left == 2 * i + 1 ? e : wd[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) wd[i] = left >= 2 * i + 2 ? wd[i] : (left == 2 * i + 1 ? wd[i] & 0xFFFFu : 0u);
+        }
         float v[16];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             v[2 * i] = __uint_as_float(wd[i] << 16);
             v[2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
         }
-        const int64_t c0 = g * kGroup + sub * 16;
         const uint32_t mb = absmax16_bits(wd);
         const bool nan = __builtin_amdgcn_ballot_w64(mb > 0x7F80u) != 0;  // wave-uniform
         if (KIND == 0) {
@@ -434,7 +269,16 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
             }
             if (!gvalid) return;
             if (sub == 0) scales[r * G + g] = sb;
-            *reinterpret_cast<uint4*>(q + r * cols + c0) = make_uint4(d[0], d[1], d[2], d[3]);
+            uint8_t* const dst = q + r * cols + c0;
+            if (!RAGGED) {
+                *reinterpret_cast<uint4*>(dst) = make_uint4(d[0], d[1], d[2], d[3]);
+            } else if (!edge || left >= 16) {
+                __builtin_memcpy(dst, d, 16);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 15; i++)
+                    if (i < left) dst[i] = uint8_t(d[i / 4] >> (8 * (i % 4)));
+            }
         } else {
             // lo = min(0, min w), hi = max(0, max w) over the group, NaN
             // skipped: without NaN fp32 min / max in any order (the zero's
@@ -491,7 +335,16 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
                 scales[r * G + g] = sb;
                 zeros[r * G + g] = uint8_t(z);
             }
-            *reinterpret_cast<uint2*>(q + (r * cols + c0) / 2) = make_uint2(d[0], d[1]);
+            uint8_t* const dst = q + (r * cols + c0) / 2;  // (cols is even)
+            if (!RAGGED) {
+                *reinterpret_cast<uint2*>(dst) = make_uint2(d[0], d[1]);
+            } else if (!edge || left >= 16) {
+                __builtin_memcpy(dst, d, 8);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 7; i++)
+                    if (2 * i < left) dst[i] = uint8_t(d[i / 4] >> (8 * (i % 4)));
+            }
         }
     };
     Cursor c0{first / octs, first % octs}, c1 = c0, c2;
@@ -555,25 +408,16 @@ __global__ __launch_bounds__(256) void embedding_kernel(QView t, const int64_t* 
 hipError_t launch_quantize(const uint16_t* w, int64_t rows, int64_t cols, int kind, uint8_t* q,
                            uint16_t* scales, uint8_t* zeros, hipStream_t stream) {
     const int64_t G = (cols + kGroup - 1) / kGroup;
-    const int64_t quads = (G + 3) / 4;
-    const int64_t waves = rows * quads;
     // enough resident waves to stream; each walks items in strides of the grid
     const int64_t cap = int64_t(device_cu_count()) * 8;
-    const unsigned grid = unsigned(std::min<int64_t>((waves + 3) / 4, cap));
-    const bool fast = cols % kGroup == 0;
-    if (fast) {
-        const int64_t octs = (G + 7) / 8;
-        const unsigned g8 = unsigned(std::min<int64_t>((rows * octs + 3) / 4, cap));
-        if (kind == 0) quantize8_kernel<0><<<g8, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-        else quantize8_kernel<1><<<g8, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-        return hipGetLastError();
-    }
-    if (kind == 0) {
-        if (fast) quantize_kernel<0, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, quads, q, scales, zeros);
-        else quantize_kernel<0, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, quads, q, scales, zeros);
+    const int64_t octs = (G + 7) / 8;
+    const unsigned grid = unsigned(std::min<int64_t>((rows * octs + 3) / 4, cap));
+    if (cols % kGroup == 0) {
+        if (kind == 0) quantize8_kernel<0, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
+        else quantize8_kernel<1, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
     } else {
-        if (fast) quantize_kernel<1, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, quads, q, scales, zeros);
-        else quantize_kernel<1, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, quads, q, scales, zeros);
+        if (kind == 0) quantize8_kernel<0, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
+        else quantize8_kernel<1, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
     }
     return hipGetLastError();
 }
