@@ -257,4 +257,14 @@ __device__ __forceinline__ float4_t sum_slices4(const float* part, int S, int64_
     return sum;
 }
 
+// The 16 bytes v, `n` bytes further on (zeros past the end).
+__device__ __forceinline__ uint4 shift_bytes(uint4 v, uint32_t n) {
+    const uint32_t b = n & 3;
+    uint32_t w0 = __builtin_amdgcn_alignbyte(v.y, v.x, b), w1 = __builtin_amdgcn_alignbyte(v.z, v.y, b);
+    uint32_t w2 = __builtin_amdgcn_alignbyte(v.w, v.z, b), w3 = __builtin_amdgcn_alignbyte(0, v.w, b);
+    if (n & 4) { w0 = w1; w1 = w2; w2 = w3; w3 = 0; }
+    if (n & 8) { w0 = w2; w1 = w3; w2 = 0; w3 = 0; }
+    return n >= 16 ? make_uint4(0, 0, 0, 0) : make_uint4(w0, w1, w2, w3);
+}
+
 }  // namespace iq
