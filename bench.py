@@ -454,7 +454,7 @@ def bench_decode_chain(torch, ops, model, steps, warmup, rows=1):
     out = {"us_per_step": round(ms * 1e3, 1), "GBps": round(wb / (ms * 1e-3) / 1e9, 1),
            "frac_hbm_peak": round(wb / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
            "rows": rows,
-           "launches": (len(step.chain.stages) if rows == 1 else 2 * len(step.chain.stages)) + 1,
+           "stages": len(step.chain.stages) + 1,
            "weight_bytes": int(wb),
            # the quantised linears of one decode step per second (attention
            # over a KV cache, sampling and the host are not in it; the

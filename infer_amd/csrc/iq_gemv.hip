@@ -46,6 +46,10 @@
 //    a separate reduce launch (gemvt_reduce_kernel / gemv_reduce_kernel)
 //    adds them in range order, so the result is deterministic and no
 //    counter has to be cleared between launches.
+//  * gemvw (5..32 rows, an even number of groups: waves that hold the split
+//    operands of a few groups in registers and stream the tiles past them):
+//    see gemvw_kernel; which calls take it, gemvw_preferred.  The kernels
+//    below serve those rows where it does not apply.
 //  * gemvh (2..32 rows, f16 split activations): see gemvh_kernel.
 //  * gemvs (7..16 rows on very wide calls, the same split operands shared
 //    through LDS by 8 tiles): see gemvs_kernel.
@@ -3162,6 +3166,10 @@ hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* con
             return e;
         }
     }
+    // From here on: 1..4 rows, and those of 5..32 that gemvw does not take
+    // (odd group counts, ragged rows, gemvw_preferred's narrow calls, partial
+    // sums beyond the workspace).  The figures compare these kernels with
+    // each other.
     if (gemvq_rows_preferred(M, total_tiles(W, n), K, n)) {
         hipError_t e = hipSuccess;
         if (launch_gemvq(x, W, bias, y, n, M, ws, stream, &e)) return e;
