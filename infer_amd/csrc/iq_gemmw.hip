@@ -262,8 +262,63 @@ __global__ __launch_bounds__(kWThreads, 2) void gemmw_kernel(const GemmwParams p
     // weights in the first steps, then the activations.
     static_assert(NW + NAT <= SB, "copies outlast the group");
     constexpr int LEAD = LO ? 2 : 1; // steps an activation read is ahead of its use
+    // 16-row blocks of this wave that hold rows of x.  In the last tile along
+    // the rows a wave may have fewer than MB: it leaves out the others'
+    // products, and its SIMD's other wave has the matrix core to itself (7B
+    // gate int8, fp32 activations at T = 201: 105 -> 103 us).  128-row tiles
+    // only: a loop beside the one below; in one loop with it, or on 256-row
+    // tiles, the accumulators of both forms do not fit the registers.
+    const int live = int(std::min<int64_t>(MB, (std::max<int64_t>(xrows - wm * 16 * MB, 0) + 15) / 16));
+    const bool less = MB == 4 && live < MB;
     uint32_t stage = 0;
-    for (int g = gbeg; g < gend; g++) {
+    for (int g = gbeg; less && g < gend; g++) {
+        const int gn = g + 1 < gend ? g + 1 : g, gz = g + 2 < gend ? g + 2 : gend - 1;
+        load_scales(gn, sn);
+        load_zeros(gz, zn);
+        const uint32_t ab = aaddr + stage;
+        // the copies, sums, conversions and barriers of the loop below, in a
+        // plain order: these waves have time to spare
+#pragma unroll
+        for (int i = 0; i < NW; i++) dma_w(gn, i);
+#pragma unroll
+        for (int i = 0; i < NAT; i++) dma_a(gn, stage ^ ASTAGE, i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int mb = 0; mb < MB - 1; mb++) {
+            if (mb >= live) continue;
+            float4_t P[4], Q[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const uint32_t ad = (ab ^ uint32_t(s << 6)) + mb * 4096;
+                const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(lds + ad);
+                const u32x4_t lo = LO ? *reinterpret_cast<const u32x4_t*>(lds + ad + APART) : hi;
+                const float4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int nb = 0; nb < 4; nb++) {
+                    const float4_t c = s == 0 ? zero : P[nb];
+                    if (LO) P[nb] = mfma16(__builtin_bit_cast(half8_t, hi), __builtin_bit_cast(half8_t, wc[nb][s]), c);
+                    else P[nb] = mfma16b(__builtin_bit_cast(bf16x8_t, hi), __builtin_bit_cast(bf16x8_t, wc[nb][s]), c);
+                    if (LO)
+                        Q[nb] = mfma16(__builtin_bit_cast(half8_t, lo), __builtin_bit_cast(half8_t, wc[nb][s]),
+                                       s == 0 ? zero : Q[nb]);
+                }
+            }
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    acc[mb][nb][r] = __builtin_fmaf(sc[nb], LO ? P[nb][r] + Q[nb][r] : P[nb][r], acc[mb][nb][r]);
+        }
+        wait_vm_only_barrier<NAT>();
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++) wc[nb][s] = convert(raw_at(nb, s), zero_of(nb));
+        wait_vm_barrier<0>();
+        take();
+        stage ^= ASTAGE;
+    }
+    for (int g = gbeg; !less && g < gend; g++) {
         const int gn = g + 1 < gend ? g + 1 : g, gz = g + 2 < gend ? g + 2 : gend - 1;
         load_scales(gn, sn);
         load_zeros(gz, zn);

@@ -100,6 +100,27 @@ def test_wide_tiles(kind, N, K, Ts):
         check_linear(y, O.bf16_to_f32(xb), W, bb, T, f"wide bf16 kind={kind} {N}x{K} T={T}")
 
 
+# Last tiles whose waves hold 1 to 3 row blocks, none, or all of them (1, 32,
+# 49 and 112 rows past a tile of 128).
+@pytest.mark.parametrize("kind", [0, 1])
+def test_wide_tiles_row_blocks(kind):
+    N, K = 18944, 3584
+    rng = np.random.default_rng(31 + kind)
+    W = QFix(rng, N, K, kind, sd=0.02)
+    for T in (129, 160, 177, 240):
+        x = rng.standard_normal((T, K), dtype=np.float32)
+        y = out_buffer(T, N)
+        say("wide tiles, row blocks", kind, N, K, T)
+        ops.launch_gemm_tiled_q(torch.from_numpy(x).cuda(), W.view, None, T, K, N, y)
+        torch.cuda.synchronize()
+        check_linear(y, x, W, None, T, f"row blocks fp32 kind={kind} T={T}")
+        xb = O.f32_to_bf16(x)
+        y = out_buffer(T, N)
+        ops.launch_gemm_bf16x(torch.from_numpy(xb.view(np.int16)).cuda(), W.view, None, T, K, N, y)
+        torch.cuda.synchronize()
+        check_linear(y, O.bf16_to_f32(xb), W, None, T, f"row blocks bf16 kind={kind} T={T}")
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 def test_wide_tiles_non_finite_rows(kind):
     """A row with inf or NaN gives a non-finite output row and leaves the
