@@ -67,13 +67,15 @@ __device__ __forceinline__ rsrc4_t rsrc4(const void* base, int64_t bytes) {
 
 // One wave's copy of 64 x 16 bytes from memory straight into LDS at
 // lds .. lds + 1023 (lane i's 16 bytes at lds + 16 i; lanes past the
-// resource's end bring zeros).  In asm, because the compiler waits for
+// resource's end bring zeros).  The whole offset is the lane's: rows past the
+// operand's last begin inside a tile, and a scalar offset is documented to be
+// outside the resource's range check.  In asm, because the compiler waits for
 // every such load before any read of LDS; wait_vm_barrier is what orders
 // them here.  No register is written, so nothing is in flight that the
 // compiler could reuse.
-__device__ __forceinline__ void dma16(rsrc4_t r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(r), "s"(soff), "s"(lds) : "memory");
+__device__ __forceinline__ void dma16(rsrc4_t r, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 :: "v"(voff), "s"(r), "s"(lds) : "memory");
 }
 
 // Waits until at most the wave's N latest memory operations are in flight
@@ -145,12 +147,12 @@ __global__ __launch_bounds__(kWThreads, 2) void gemmw_kernel(const GemmwParams p
                                      : uint32_t((lane >> 3) * row_bytes) + uint32_t(((lane & 7) ^ (lane >> 4)) << 4);
     auto dma_w = [&](int g, int i) {
         const int j = wave * NW + i;
-        dma16(rw, KIND == 1 ? wvoff : wvoff ^ uint32_t((i & 1) << 6),
-              uint32_t(j * (1024 / WROW) * row_bytes + int64_t(g) * WROW), lds0 + WBASE + uint32_t(j) * 1024);
+        dma16(rw, (KIND == 1 ? wvoff : wvoff ^ uint32_t((i & 1) << 6)) +
+                      uint32_t(j * (1024 / WROW) * row_bytes + int64_t(g) * WROW), lds0 + WBASE + uint32_t(j) * 1024);
     };
     auto dma_a = [&](int g, uint32_t stage, int i) {
         const int part = i / NA, j = wave * NA + i % NA;
-        dma16(part ? ral : ra, avoff ^ uint32_t((i & 3) << 6), uint32_t(int64_t(j) * 8 * p.K + int64_t(g) * 256),
+        dma16(part ? ral : ra, (avoff ^ uint32_t((i & 3) << 6)) + uint32_t(int64_t(j) * 8 * p.K + int64_t(g) * 256),
               lds0 + stage + part * APART + uint32_t(j) * 1024);
     };
     constexpr int NAT = NA * PARTS;
@@ -173,12 +175,12 @@ __global__ __launch_bounds__(kWThreads, 2) void gemmw_kernel(const GemmwParams p
     auto load_scales = [&](int g, uint16_t (&s)[4]) {
 #pragma unroll
         for (int nb = 0; nb < 4; nb++)
-            s[nb] = __builtin_amdgcn_raw_buffer_load_b16(rsc, soff * 2, uint32_t(nb * 16 * p.G + g) * 2, 0);
+            s[nb] = __builtin_amdgcn_raw_buffer_load_b16(rsc, (soff + uint32_t(nb * 16 * p.G + g)) * 2, 0, 0);
     };
     auto load_zeros = [&](int g, uint32_t (&z)[4]) {
 #pragma unroll
         for (int nb = 0; nb < 4; nb++)
-            z[nb] = KIND == 1 ? __builtin_amdgcn_raw_buffer_load_b8(rzp, soff, uint32_t(nb * 16 * p.G + g), 0) : 0u;
+            z[nb] = KIND == 1 ? __builtin_amdgcn_raw_buffer_load_b8(rzp, soff + uint32_t(nb * 16 * p.G + g), 0, 0) : 0u;
     };
 
     // Converted weights of the current group: [16-column block][32-column k step]
