@@ -201,7 +201,10 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
         else off = g < G ? uint32_t((g * kGroup + sub * 16) * 2) : kOob;
         Raw x;
         x.a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
-        x.b = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 16, 0));
+        // (added to the lane's offset, not as the scalar offset, which is
+        // documented to be outside the range check: these 16 bytes can be
+        // the first past the matrix)
+        x.b = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off + 16, 0, 0));
         return x;
     };
     auto process = [&](const Cursor& cc, const Raw& cur) {

@@ -31,7 +31,7 @@ def arguments(text, start):
     raise AssertionError("unbalanced call")
 
 
-@pytest.mark.parametrize("name", ["iq_gemmw.hip"])
+@pytest.mark.parametrize("name", ["iq_gemmw.hip", "iq_quant.hip"])
 def test_requests_are_range_checked_whole(name):
     with open(os.path.join(CSRC, name)) as f:
         text = re.sub(r"//[^\n]*", "", f.read())
