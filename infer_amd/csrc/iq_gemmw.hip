@@ -75,7 +75,7 @@ __device__ __forceinline__ rsrc4_t rsrc4(const void* base, int64_t bytes) {
 // compiler could reuse.
 __device__ __forceinline__ void dma16(rsrc4_t r, uint32_t voff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-                 :: "v"(voff), "s"(r), "s"(lds) : "memory");
+                 :: "v"(voff), "s"(r), "s"(lds) : "memory", "m0");
 }
 
 // Waits until at most the wave's N latest memory operations are in flight

@@ -1,8 +1,9 @@
-"""CPU check of the kernels whose memory requests may start inside an operand
-and reach past its end: the buffer resource's range check compares the vector
-offset (and the instruction's constant) with the operand's size, and the
-scalar offset is documented to be outside of it, so every request of these
-sources carries its whole offset in the vector part."""
+"""CPU checks of the kernels' source text.  Requests that may start inside an
+operand and reach past its end: the buffer resource's range check compares the
+vector offset (and the instruction's constant) with the operand's size, and
+the scalar offset is documented to be outside of it, so every request of these
+sources carries its whole offset in the vector part.  And inline assembly
+names the registers it writes."""
 import os
 import re
 
@@ -44,3 +45,15 @@ def test_requests_are_range_checked_whole(name):
     for a in asm:
         assert re.match(r"buffer_load_\w+ %\d+, %\d+, 0 offen", a), f"{name}: scalar offset in {a!r}"
     assert calls or asm
+
+
+def test_asm_that_writes_m0_says_so():
+    for name in sorted(os.listdir(CSRC)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        with open(os.path.join(CSRC, name)) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        for m in re.finditer(r"asm(?:\s+volatile)?\s*\(", text):
+            call = text[m.end() - 1:text.index(";", m.end())]
+            if re.search(r"\bm0,", call):
+                assert '"m0"' in call, f"{name}: {call}"
