@@ -83,7 +83,9 @@ inline GemmwPlan gemmw_plan(int64_t T, int64_t N, int64_t G, int bm, bool lo, in
     pl.tiles_m = int((T + bm - 1) / bm);
     pl.tiles_n = int((N + 255) / 256);
     const int64_t tiles = int64_t(pl.tiles_m) * pl.tiles_n;
-    if (tiles > (1 << 24)) return pl;
+    // (a tile's byte offsets are 32 bits wide: 256 rows of 2 K bytes stay
+    // below 2^31 for K < 2^22)
+    if (tiles > (1 << 24) || G >= (1 << 15)) return pl;
     pl.full = least > 1 ? 0 : int(tiles / cus * cus);
     pl.gch = int(G);
     const int64_t tail = tiles - pl.full;

@@ -48,6 +48,15 @@ int main() {
                                     }
                                     if (least > 1 && G >= least) CHECK(p.splits >= 2);
                                 }
+    // rows so long that a tile's 32-bit byte offsets would wrap are refused
+    for (int G : {1 << 15, 1 << 16, (1 << 17) - 1})
+        for (int T : {65, 300, 1024})
+            for (int64_t N : {int64_t(4096), int64_t(8192)})
+                for (int bm : {128, 256}) {
+                    const int lo = 0, cus = 256, least = 1;
+                    const int64_t part = int64_t(16) << 20;
+                    CHECK(int64_t(bm) * G * 256 < (int64_t(1) << 31) || iq::gemmw_plan(T, N, G, bm, lo, cus, part, least).us > 1e29);
+                }
     std::printf("%ld plans checked, %ld split, %ld refused, %d failures\n", plans, split, none, failures);
     return failures ? 1 : 0;
 }
