@@ -3,6 +3,7 @@
 #pragma once
 
 #include "iq_internal.h"
+#include "iq_plan.h"
 
 namespace iq {
 
@@ -22,8 +23,7 @@ struct GemmwParams {
     int splits, gch;     // K ranges of the others, groups per range
 };
 
-// Runs the wide-tile GEMM if it is estimated to take at most other_us (the
-// estimate for the narrower tiles); false: nothing launched.
-bool launch_gemmw(GemmwParams p, int kind, double other_us, int64_t part_floats, hipStream_t stream);
+// The wide-tile GEMM with the tiles and K ranges of pl (gemmw_choose).
+hipError_t launch_gemmw(GemmwParams p, int kind, const GemmwPlan& pl, hipStream_t stream);
 
 }  // namespace iq

@@ -902,49 +902,11 @@ void launch_gemm_t(const GemmParams& p, int mode, int bm, hipStream_t stream) {
     else gemm_kernel<KIND, XF32, kAligned, NJ, 128><<<grid, kThreads, 0, stream>>>(p);
 }
 
-// Few output tiles (short T): split K into ranges of whole 128-column groups
-// so that the tiles x ranges fill the workgroup slots of the CUs (per_cu
-// resident workgroups of the instance per CU) in one round, the range sums
-// added by gemm_reduce_kernel; needs room for the sums.  Rounding the range count down rather than up keeps a second,
-// mostly idle round of workgroups off the critical path (7B down 3584 x
-// 18944 at T = 80 / 200, fp32 activations: 76.8 / 140.6 -> 60.7 / 111.0
-// us; bf16 activations 50.1 / 94.9 -> 36.6 / 69.4 us; 7B gate 18944 x 3584
-// with bf16 activations at T = 17..48, on the three-term kernel's one
-// workgroup per CU: 29.5..32.6 -> 24.1..27.0 us).  The exception: tiles
-// that fill only half to two thirds of one round, on rows of at least 24
-// groups, take 3 ranges (two full rounds of shorter workgroups; 7B gate at
-// T = 65 / 96 / 128, int8, fp32 activations 78.0 / 72.9 / 73.3 -> 66.4 /
-// 64.9 / 68.7 us, bf16 activations 49.6 / 49.7 / 50.2 -> 41.8 / 43.8 /
-// 46.5 us, int4 8-16 % faster; 1.5B gate 8960 x 1536, 12 groups, at T =
-// 256 lost 38.2 -> 44.5 us), and so do tiles that fill one round up to 2.5
-// rounds (7B gate at T = 256, int8 / int4: fp32 activations 125.9 / 119.8
-// -> 116.3 / 107.5 us, bf16 84.9 / 95.9 -> 81.8 / 88.9 us; wider ones
-// overrun the partial sums).  part_floats: the workspace's partial-sum
-// capacity.
-int pick_splits(int tiles, int slots, int64_t G, int64_t T, int64_t N, int64_t part_floats) {
-    if (G < 2) return 1;
-    if (tiles >= slots) {
-        if (2 * tiles < 5 * slots && G >= 24 && 3 * T * N <= part_floats) return 3;
-        return 1;
-    }
-    int S = slots / tiles;
-    S = S > 16 ? 16 : S;
-    while (S > 1 && int64_t(S) * T * N > part_floats) S--;
-    if (S == 1 && 3 * tiles <= 2 * slots && G >= 24 && 3 * T * N <= part_floats) S = 3;
-    return S;
-}
-
 void plan_splits(GemmParams& p, int64_t part_floats, int per_cu) {
-    p.splits = 1;
-    p.kchunk = p.K;
-    const int tiles = p.tiles_m * p.tiles_n, want = per_cu * device_cu_count();
-    if (!p.part) return;
-    const int64_t G = p.G;
-    const int S = pick_splits(tiles, want, G, p.T, p.N, part_floats);
-    if (S < 2 || G < 2) return;
-    const int64_t gch = (G + S - 1) / S;
-    p.kchunk = gch * kGroup;
-    p.splits = int((G + gch - 1) / gch);
+    const int S = pick_splits(p.tiles_m * p.tiles_n, per_cu * device_cu_count(), p.G, p.T, p.N, p.part ? part_floats : 0);
+    const KRanges r = k_ranges(S, p.G);
+    p.splits = r.splits;
+    p.kchunk = r.splits > 1 ? r.gch * kGroup : p.K;
 }
 
 template <int KIND, bool XF32>
@@ -981,22 +943,6 @@ void launch_gemm_nj(GemmParams& p, int mode, int bm, int64_t part_floats, hipStr
     }
 }
 
-// Estimated time of tiles x S K ranges on the narrow tiles, workgroups of
-// which per_cu share a CU, group_us a group and round (measured: 7B gate
-// 18944 x 3584, T = 201 and 384..1024), plus the range sums' way through
-// memory: what the wide tiles' estimate is compared with (GemmwPlan).  Both
-// sides at the line, fp32 int8: 7B gate at T = 160 / 201 86 / 120 -> 86
-// (kept) / 105 us, o 3584 x 3584 at T = 384 / 512 47 / 55 -> 46 / 52, 1.5B
-// gate 8960 x 1536 at T = 384 / 512 45 (kept) / 66 -> 44 / 57; bf16: 7B gate
-// at T = 300 / 384 80 / 83 (kept) against 88 / 112 on the wide tiles, at T =
-// 450 133 -> 113.
-double narrow_us(int tiles, int per_cu, int S, int64_t G, int64_t T, int64_t N, double group_us) {
-    const int slots = per_cu * device_cu_count();
-    const int64_t gch = (G + S - 1) / S;
-    return 4.0 + double((int64_t(tiles) * S + slots - 1) / slots) * double(gch) * group_us +
-           (S > 1 ? 5.0 + double(S) * double(T) * double(N) * 8 / 9e6 : 0.0);
-}
-
 // The fp16 operand path (K % 128 == 0, 16-byte aligned activations): one
 // preparation launch, the GEMM, and the range sums when K is split, for T
 // rows whose operands fit the workspace's operand area.
@@ -1027,46 +973,24 @@ hipError_t launch_gemmh_chunk(const float* x_f32, const QView& W, const uint16_t
     p.q = W.q; p.scales = W.scales; p.zeros = W.zeros; p.bias = bias; p.y = y;
     p.T = T; p.N = W.rows; p.K = K; p.G = W.groups;
     p.part = ws->partials;
-    // 64 x 128 tiles on 4 waves, two workgroups per CU (a 4-wave workgroup
-    // of 128 rows, whose hi + lo operand buffers fill the LDS, runs alone
-    // on its CU: 7B int8 at T = 128 / 512 / 1024, down 3584 x 18944 99 /
-    // 334 / 684 -> 66 / 212 / 433 us, gate 18944 x 3584 266 / 440 -> 201 /
-    // 393 us at 512 / 1024, o 3584 x 3584 at 1024 142 -> 93 us).  From T =
-    // 512, int4 and rows of K >= 2048 take 128 x 128 tiles on 8 waves, each
-    // converted weight tile feeding twice the rows: 7B int4 at T = 1024 /
-    // 2048 down 426 / 936 -> 378 / 782 us, gate 389 / 801 -> 354 / 721 us,
-    // int8 gate 402 -> 381 us at 1024 (1.5B int8 gate 8960 x 1536: 110 ->
-    // 116 us, kept at 64 rows).
-    const bool wide_t = T >= 512 && (W.kind == 1 || K >= 2048);
-    const int bm = wide_t ? 128 : 64;
+    const int bm = gemmh_rows(T, K, W.kind);
     p.tiles_m = int((T + bm - 1) / bm);
     p.tiles_n = int((p.N + 127) / 128);
-    // K ranges (pick_splits)
-    p.splits = 1;
-    p.kchunk = K;
-    {
-        // (as plan_splits: 1.5B o 1536 x 1536 at T = 80 / 256 18.5 / 23.0
-        // -> 13.6 / 16.5 us)
-        const int tiles = p.tiles_m * p.tiles_n, want = (bm == 128 ? 1 : 2) * device_cu_count();
-        const int64_t G = K / kGroup;
-        if (G >= 2) {
-            const int S = pick_splits(tiles, want, G, T, p.N, ws->part_floats);
-            if (S >= 2) {
-                const int64_t gch = (G + S - 1) / S;
-                p.kchunk = gch * kGroup;
-                p.splits = int((G + gch - 1) / gch);
-            }
+    // K ranges (1.5B o 1536 x 1536 at T = 80 / 256 18.5 / 23.0 -> 13.6 / 16.5
+    // us)
+    const KRanges r = k_ranges(pick_splits(p.tiles_m * p.tiles_n, (bm == 128 ? 1 : 2) * device_cu_count(), W.groups, T, p.N,
+                                           ws->part_floats), W.groups);
+    p.splits = r.splits;
+    p.kchunk = r.splits > 1 ? r.gch * kGroup : K;
+    if (reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
+        const GemmwPlan wide = gemmw_choose(T, p.N, K, W.kind, true, device_cu_count(), ws->part_floats);
+        if (wide.us < 1e29) {
+            GemmwParams w;
+            w.a = reinterpret_cast<const uint16_t*>(ah); w.al = reinterpret_cast<const uint16_t*>(al); w.rs = rs;
+            w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
+            w.T = T; w.N = W.rows; w.K = K; w.G = W.groups;
+            return launch_gemmw(w, W.kind, wide, stream);
         }
-    }
-    if (T > 64 && reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
-        GemmwParams w;
-        w.a = reinterpret_cast<const uint16_t*>(ah); w.al = reinterpret_cast<const uint16_t*>(al); w.rs = rs;
-        w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
-        w.T = T; w.N = W.rows; w.K = K; w.G = W.groups;
-        if (launch_gemmw(w, W.kind, narrow_us(p.tiles_m * p.tiles_n, bm == 128 ? 1 : 2, p.splits, W.groups, T, p.N,
-                                              bm == 128 ? (W.kind == 1 ? 2.45 : 2.65) : (W.kind == 1 ? 2.05 : 2.4)),
-                         ws->part_floats, stream))
-            return hipGetLastError();
     }
     const unsigned ggrid = unsigned(p.tiles_m * p.tiles_n * p.splits);
     if (bm == 128) {
@@ -1111,30 +1035,14 @@ hipError_t launch_gemm(const float* x_f32, const uint16_t* x_bf16, const QView& 
                        const uint16_t* bias, int64_t T, float* y, Workspace* ws, hipStream_t stream) {
     {
         const uintptr_t xa = x_f32 ? reinterpret_cast<uintptr_t>(x_f32) : reinterpret_cast<uintptr_t>(x_bf16);
-        // fp32 activations: 17..32 rows of wide or long-K matrices on
-        // gemvq's row blocks; past 32 rows on whole 128-column groups the
-        // fp16 operand path (22 significant bits against the 24 of three
-        // bf16 terms at 1.5x the MFMAs, and faster: 7B at T = 1024, gate
-        // 18944 x 3584 int4 648 -> 440 us, down 1053 -> 681 us); up to 32
-        // rows the three-term split inside gemm_kernel, whose single launch
-        // beats the preparation launch on the narrower matrices left here
-        // (1.5B at 32 rows: o 1536 x 1536 16.9 -> 11.6 us, down 1536 x 8960
-        // 25.4 -> 21.8; 7B o 22.9 either way), and so up to 64 rows on
-        // matrices of at most 2^24 weights (T = 64: 1.5B o 15.6 -> 10.2, down
-        // 24.1 -> 19.7, 7B o 23.7 -> 21.4 us; 7B gate 44.8 against 64.7) and
-        // up to 256 rows on matrices of at most 2^22 (T = 96..256: 7B k 512
-        // x 3584 18.0..22.4 -> 13.3..14.6 us, 1.5B o 23.2..25.1 ->
-        // 17.7..22.4), at any T on matrices of at most 2^19 (1.5B k 256 x
-        // 1536 at T = 257 / 512 / 2048: 17.3 / 20.7 / 34.0 -> 12.7 / 12.4 /
-        // 25.9 us)
+        // fp32 activations: 17..32 rows of wide or long-K matrices on the rows
+        // GEMV, then the prepared fp16 operands where gemm_kernel does not split
+        // x itself
         if (x_f32) {
             hipError_t e = hipSuccess;
             if (launch_gemm_rows(x_f32, W, bias, T, y, ws, stream, &e)) return e;
         }
-        const int64_t nk = W.rows * W.cols;
-        const bool split_in_kernel = T <= 32 || (T <= 64 && nk <= (int64_t(1) << 24)) ||
-                                     (T <= 256 && nk <= (int64_t(1) << 22)) || nk <= (int64_t(1) << 19);
-        if (x_f32 && !split_in_kernel && W.cols % kGroup == 0 && xa % 16 == 0)
+        if (x_f32 && !gemm_splits_x(T, W.rows, W.cols) && W.cols % kGroup == 0 && xa % 16 == 0)
             return launch_gemmh(x_f32, W, bias, T, y, ws, stream);
     }
     GemmParams p;
@@ -1148,30 +1056,16 @@ hipError_t launch_gemm(const float* x_f32, const uint16_t* x_bf16, const QView& 
     const int64_t least = W.kind == 1 ? 32 : 16;
     const int mode = p.K % kGroup == 0 && xa % 16 == 0 ? kAligned
                      : p.K >= least && p.K < (int64_t(1) << 22) ? kUnaligned : kBytes;
-    // 64-row tiles for short T (less MFMA work on padding rows, more tiles):
-    // 7B int8, fp32 activations, gate 18944 x 3584 at T = 33 / 64 / 128 /
-    // 256: 115 / 113 / 137 / 202 -> 55 / 58 / 97 / 139 us; down 3584 x
-    // 18944 at T = 64 / 256: 115 / 186 -> 58 / 170 us, but at T = 128 (a
-    // narrow matrix, already split over K) 93 -> 103: kept at 128 rows there
-    const bool short_t = T <= 64 || (T > 128 && T <= 256) || (T <= 128 && W.rows >= 8192);
-    // 256-row tiles (8 waves) for long bf16 prefills of narrow int4
-    // matrices: each dequantised weight tile (nibble unpack + zero point,
-    // the costlier conversion) feeds twice the MFMAs.  7B at T = 1024 with
-    // 256 / 128 rows: int4 down 259 / 275 us, int4 gate|up 235 / 208 us,
-    // int8 down 269 / 249 us (one 8-wave workgroup per CU leaves the step
-    // barriers uncovered, which costs more than the conversion saves on a
-    // wide matrix or with int8's cheaper conversion).
-    const bool big = !x_f32 && mode == kAligned && T >= 512 && W.kind == 1 && W.rows < 8192;
-    const int bm = (short_t && mode != kBytes) ? 64 : (big ? 256 : 128);
-    if (!x_f32 && mode == kAligned && T > 64 && reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
-        GemmwParams w;
-        w.a = x_bf16; w.al = nullptr; w.rs = nullptr;
-        w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
-        w.T = T; w.N = W.rows; w.K = p.K; w.G = W.groups;
-        const int rows = bm == 256 ? 128 : bm, tiles = int((T + rows - 1) / rows) * int((p.N + 127) / 128);
-        const int S = pick_splits(tiles, 2 * device_cu_count(), p.G, T, p.N, ws->part_floats);
-        if (launch_gemmw(w, W.kind, narrow_us(tiles, 2, S, p.G, T, p.N, bm == 64 ? 1.9 : 2.8), ws->part_floats, stream))
-            return hipGetLastError();
+    const int bm = mode == kBytes ? 128 : gemm_rows(T, W.rows, W.kind, !x_f32 && mode == kAligned);
+    if (!x_f32 && mode == kAligned && reinterpret_cast<uintptr_t>(W.q) % 16 == 0) {
+        const GemmwPlan wide = gemmw_choose(T, p.N, p.K, W.kind, false, device_cu_count(), ws->part_floats);
+        if (wide.us < 1e29) {
+            GemmwParams w;
+            w.a = x_bf16; w.al = nullptr; w.rs = nullptr;
+            w.q = W.q; w.scales = W.scales; w.zeros = W.zeros; w.bias = bias; w.y = y; w.part = ws->partials;
+            w.T = T; w.N = W.rows; w.K = p.K; w.G = W.groups;
+            return launch_gemmw(w, W.kind, wide, stream);
+        }
     }
     p.tiles_m = int((T + bm - 1) / bm);
     if (x_f32) {

@@ -455,25 +455,13 @@ void launch_t(const GemmwParams& p, hipStream_t stream) {
 
 }  // namespace
 
-bool launch_gemmw(GemmwParams p, int kind, double other_us, int64_t part_floats, hipStream_t stream) {
-    const bool lo = p.al != nullptr;
-    // (bf16 rows of at least 24 groups at T <= 256 keep the three or more
-    // ranges, and with them the shorter sums, that the narrow tiles have)
-    const int least = !lo && p.T <= 256 && p.G >= 24 ? 3 : 1;
-    const int cus = device_cu_count();
-    GemmwPlan pl = gemmw_plan(p.T, p.N, p.G, 128, lo, cus, part_floats, least);
-    if (!lo) {
-        const GemmwPlan p8 = gemmw_plan(p.T, p.N, p.G, 256, lo, cus, part_floats, least);
-        if (p8.us < pl.us) pl = p8;
-    }
-    // (the estimates are good to some percent: 5 % in doubt for what is there)
-    if (pl.us > 0.95 * other_us) return false;
+hipError_t launch_gemmw(GemmwParams p, int kind, const GemmwPlan& pl, hipStream_t stream) {
     p.tiles_m = pl.tiles_m;
     p.tiles_n = pl.tiles_n;
     p.full = pl.full;
     p.splits = pl.splits;
     p.gch = pl.gch;
-    if (lo) {
+    if (p.al) {
         if (kind == 1) launch_t<1, true, 4>(p, stream);
         else launch_t<0, true, 4>(p, stream);
     } else if (pl.bm == 256) {
@@ -483,7 +471,7 @@ bool launch_gemmw(GemmwParams p, int kind, double other_us, int64_t part_floats,
         if (kind == 1) launch_t<1, false, 4>(p, stream);
         else launch_t<0, false, 4>(p, stream);
     }
-    return true;
+    return hipGetLastError();
 }
 
 }  // namespace iq

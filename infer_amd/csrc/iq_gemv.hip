@@ -1134,19 +1134,6 @@ size_t gemv1_lds(int64_t G, int R, bool half = false) {
     return size_t(G) * ((half ? R / 2 : (R < 4 ? R : 4)) * kLimbRec + R * 16);
 }
 
-// 1..4 rows always; 5..8 rows (two blocks of 4, the second converted after
-// the first is multiplied) only on narrow launches, measured at 7B: o (224
-// tiles) 10.1 -> 9.2 us at 8 rows and q|k|v (288) 12.2 -> 10.5 at 5, but
-// q|k|v 12.2 -> 13.1 at 8 rows and gate|up 35 -> 41 / 53 us at 5 / 8.
-bool gemv1_rows_preferred(int M, int tiles, int64_t G) {
-    if (M <= 4) return true;
-    if (M > 8) return false;
-    const int cus = device_cu_count();
-    // short rows convert fast: 1.5B gate (G = 12, 560 tiles) at 7 / 8 rows
-    // 11.7 -> 10.1 / 11.8 -> 10.7 us (int8)
-    return tiles <= cus || (tiles < 4 * cus && (M <= 6 || G <= 16));
-}
-
 // Shape of a 1-row launch: groups per wave slice (gs), waves per workgroup
 // (ks), the slice capacity NG of the kernel instance (0: not applicable),
 // the grid (kr workgroups per 16-row tile, each a K range of gr groups).
@@ -2731,54 +2718,6 @@ void launch_gemvw_k(const GemvParams& p, int ng, unsigned grid, int nw, hipStrea
     }
 }
 
-// gemvw's ranges and workgroups for M rows, `units` 16-row tiles (or SwiGLU
-// pairs of them): S ranges of gs groups, nw waves of ng groups a workgroup,
-// nrb workgroups a range.  ok: G is whole sets of ng groups.
-struct GwPlan {
-    int ng = 0, S = 0, gs = 0, nw = 0, nrb = 0;
-    bool ok = false;
-};
-
-GwPlan gemvw_plan(int64_t G, int M, int units) {
-    GwPlan pl;
-    // groups a wave: 4 (2 from 17 rows: their operands fill the registers),
-    // or 2 where G leaves a remainder and on short rows, whose few waves
-    // would otherwise leave half the CU's registers unused (1.5B gate|up, G =
-    // 12, at 16 rows int4 / int8 14.0 / 15.0 -> 10.9 / 11.6 us, 5 rows 10.7
-    // / 12.1 -> 10.3 / 10.2); whole sets only
-    pl.ng = M <= 16 && G % 4 == 0 && G > 16 ? 4 : 2;
-    if (M < 5 || M > kMaxRowsGemv || G % pl.ng) return pl;
-    pl.S = int((G + 8 * pl.ng - 1) / (8 * pl.ng));
-    pl.gs = int((G + pl.S - 1) / pl.S);
-    pl.gs = (pl.gs + pl.ng - 1) / pl.ng * pl.ng;
-    pl.S = int((G + pl.gs - 1) / pl.gs);
-    pl.nw = pl.gs / pl.ng;
-    const int slots = device_cu_count() * (8 / pl.nw);
-    pl.nrb = std::min(units, std::max(1, slots / pl.S));
-    // (one or two tiles a workgroup: two each, so that no CU waits for a
-    // second workgroup)
-    if (units < 2 * pl.nrb && units > pl.nrb) pl.nrb = (units + 1) / 2;
-    pl.ok = true;
-    return pl;
-}
-
-// gemvw or the other kernels (both measured in a graph, us, others -> gemvw):
-// 17..32 rows from 64 tiles on (7B k 512 x 3584 at 17 rows 11.2 kept against
-// 11.4; 1024 x 7168 16.9 -> 12.6); 9..16 rows on long rows (1.5B down, G =
-// 70, int8 20.9 -> 11.0, int4 15.2 -> 10.2) or where tiles x groups fill the
-// card (7B q|k|v, 288 x 28, 12.3 -> 11.4; o, 224 x 28, int4 9.7 kept against
-// 10.4, int8 11.9 -> 11.1; 7168 x 1024, 448 x 8, 7.6 kept against 8.9); 5..8
-// rows wherever the 1-row kernel's exact integer sums do not serve (on those
-// narrow calls, where gemvw would be up to 25 % faster at 8 rows, its error
-// is 1.2 to 1.4 times theirs).
-bool gemvw_preferred(int M, int tiles, int64_t K, int kind) {
-    const int64_t G = K / kGroup;
-    if (M < 5 || M > kMaxRowsGemv || K % kGroup || G % 2) return false;
-    if (M > 16) return tiles >= 64;
-    if (M > 8) return G >= 48 || tiles * G >= (kind == 1 ? 6400 : 6000);
-    return tiles >= 1024 || G >= 128 || !gemv1_rows_preferred(M, tiles, G);
-}
-
 // gemvw on n matrices straight from x (false: G has no whole sets of
 // groups, or the partial sums would not fit).
 bool launch_gemvw(const float* x, const QView* W, const uint16_t* const* bias, float* const* y, int n, int M, Workspace* ws,
@@ -2789,7 +2728,7 @@ bool launch_gemvw(const float* x, const QView* W, const uint16_t* const* bias, f
         p.mat[i] = MatRef{W[i].q, W[i].scales, W[i].zeros, bias[i], y[i], W[i].rows, tiles};
         tiles += int((W[i].rows + 15) / 16);
     }
-    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles);
+    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles, device_cu_count());
     if (!pl.ok || (pl.S > 1 && int64_t(pl.S) * M * tiles * 16 > ws->part_floats)) return false;
     p.nmat = n;
     p.K = W[0].cols;
@@ -3154,7 +3093,7 @@ hipError_t launch_gemv_prepped(const QView& W, const uint16_t* bias, int M, floa
 hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* const* bias, float* const* y,
                              int n, int M, Workspace* ws, hipStream_t stream) {
     const int64_t K = W[0].cols, G = W[0].groups;
-    if (gemvw_preferred(M, total_tiles(W, n), K, W[0].kind)) {
+    if (gemvw_preferred(M, total_tiles(W, n), K, W[0].kind, device_cu_count())) {
         hipError_t e = hipSuccess;
         if (launch_gemvw(x, W, bias, y, n, M, ws, stream, &e)) {
             // gemvw leaves a preparation's buffers alone, but callers may
@@ -3236,7 +3175,7 @@ hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* con
         if (e != hipSuccess) return e;
         return launch_gemvh(W, bias, y, n, M, ws, stream);
     }
-    if (gemv1_rows_preferred(M, total_tiles(W, n), G)) {
+    if (gemv1_rows_preferred(M, total_tiles(W, n), G, device_cu_count())) {
         // the 1-row kernel converts x itself; 2..8 rows share each weight
         // operand (no preparation launch, and the workspace's preparation
         // stays as it was)
@@ -3297,7 +3236,7 @@ hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* con
 bool launch_gemm_rows(const float* x, const QView& W, const uint16_t* bias, int64_t T, float* y, Workspace* ws,
                       hipStream_t stream, hipError_t* err) {
     const int tiles = int((W.rows + 15) / 16);
-    if (T > 16 && T <= kMaxRowsGemv && gemvw_preferred(int(T), tiles, W.cols, W.kind) &&
+    if (T > 16 && T <= kMaxRowsGemv && gemvw_preferred(int(T), tiles, W.cols, W.kind, device_cu_count()) &&
         launch_gemvw(x, &W, &bias, &y, 1, int(T), ws, stream, err))
         return true;
     if (!gemvq_rows_preferred(T, tiles, W.cols, 1)) return false;
@@ -3341,7 +3280,7 @@ RowsSetup rows_setup(const QView* W, int n, int M, int64_t part_floats) {
     r.p.ntiles = tiles;
     r.p.to_part = 1;
     const int cus = device_cu_count();
-    r.w = gemvw_plan(G, M, tiles);
+    r.w = gemvw_plan(G, M, tiles, cus);
     if (r.w.ok && int64_t(r.w.S) * M * tiles * 16 <= part_floats) {
         r.p.gs = r.w.gs;
         r.p.S = r.w.S;
@@ -3457,7 +3396,7 @@ hipError_t launch_chain_rows(const QView* W, int n, int M, const RowsIn& in, flo
 
 bool chain_w_applies(const QView* W, int n, int M, bool pair) {
     const int tiles = pair ? int((W[0].rows + 15) / 16) : total_tiles(W, n);
-    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles);
+    const GwPlan pl = gemvw_plan(W[0].groups, M, tiles, device_cu_count());
     return pl.ok && pl.S == 1;
 }
 
@@ -3469,7 +3408,7 @@ hipError_t launch_chain_w(const QView* W, int n, int M, const RowsIn& in, const 
         p.mat[i] = MatRef{W[i].q, W[i].scales, W[i].zeros, bias[i], pair ? y[0] : y[i], W[i].rows, tiles};
         tiles += int((W[i].rows + 15) / 16);
     }
-    const GwPlan pl = gemvw_plan(W[0].groups, M, pair ? tiles / 2 : tiles);
+    const GwPlan pl = gemvw_plan(W[0].groups, M, pair ? tiles / 2 : tiles, device_cu_count());
     if (!pl.ok || pl.S != 1) return hipErrorInvalidValue;
     p.nmat = n;
     p.K = W[0].cols;

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "iq_device.h"
+#include "iq_plan.h"
 
 namespace iq {
 
@@ -52,7 +53,6 @@ struct Workspace {
     }
 };
 
-constexpr int kMaxRowsGemv = 32;            // GpuBatch::kMaxRows (kernels/batch_gpu.h:80)
 constexpr int64_t kMaxKp = 131072;          // padded K limit of the GEMV
 constexpr int64_t kPartialFloats = int64_t(4) << 20;  // 16 MiB of split-K partials (every workspace)
 constexpr int64_t kStreamPartialFloats = int64_t(16) << 20;  // 64 MiB in a per-stream workspace

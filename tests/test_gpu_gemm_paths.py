@@ -8,6 +8,7 @@ import torch
 from infer_amd import ops
 from oracle import oracle as O
 from tests.gpu_util import QFix, bias_of, check_linear, out_buffer, say
+from tests.test_gpu_routes import Packed, check_sampled
 
 pytestmark = pytest.mark.gpu
 
@@ -77,9 +78,13 @@ def test_unaligned_rows_ignore_what_follows(kind):
 # tiles of fp32 activations, all K ranges of split tiles, rows and columns
 # past the last tile, N that is no multiple of 4 (the reduction's scalar
 # stores); whole rounds of tiles beside split ones are in test_gpu_routes
-# (the 7B gate at T = 1024).
+# (the 7B gate at T = 1024).  Which of these calls the wide tiles serve is
+# in test_routes.py.
+WIDE = [(18947, 3584, (100, 201)), (3587, 18944, (257, 450)), (8192, 4096, (513,))]
+
+
 @pytest.mark.parametrize("kind", [0, 1])
-@pytest.mark.parametrize("N,K,Ts", [(18947, 3584, (100, 201)), (3587, 18944, (257, 450)), (8192, 4096, (513,))])
+@pytest.mark.parametrize("N,K,Ts", WIDE)
 def test_wide_tiles(kind, N, K, Ts):
     rng = np.random.default_rng(N + kind)
     W = QFix(rng, N, K, kind, sd=0.02)
@@ -100,8 +105,9 @@ def test_wide_tiles(kind, N, K, Ts):
         check_linear(y, O.bf16_to_f32(xb), W, bb, T, f"wide bf16 kind={kind} {N}x{K} T={T}")
 
 
-# Last tiles whose waves hold 1 to 3 row blocks, none, or all of them (1, 32,
-# 49 and 112 rows past a tile of 128).
+# Row counts around the one from which the 7B gate takes wide tiles: 129, 160
+# and 177 stay on the narrow ones, 240 takes wide tiles but for int4 with
+# fp32 activations (3 row blocks in the last tile's second wave).
 @pytest.mark.parametrize("kind", [0, 1])
 def test_wide_tiles_row_blocks(kind):
     N, K = 18944, 3584
@@ -121,17 +127,49 @@ def test_wide_tiles_row_blocks(kind):
         check_linear(y, O.bf16_to_f32(xb), W, None, T, f"row blocks bf16 kind={kind} T={T}")
 
 
+# Row counts with 1, 2 or 3 of the 4 row blocks of the last 128-row tile's
+# first wave in use and none of its second, and all and 1, 2 or 3, for both
+# kinds and activation types (test_routes.py asserts it); bf16 at T = 600 and
+# 700 the same on 256-row tiles.
+LAST_BLOCKS = (18947, 3584, (400, 410, 430, 450, 470, 490, 600, 700))
+
+
 @pytest.mark.parametrize("kind", [0, 1])
-def test_wide_tiles_non_finite_rows(kind):
+@pytest.mark.parametrize("T", LAST_BLOCKS[2])
+def test_wide_tiles_last_row_blocks(kind, T):
+    N, K, _ = LAST_BLOCKS
+    rng = np.random.default_rng(47 + 2 * T + kind)
+    W = Packed(rng, N, K, kind)
+    bb, bd = bias_of(rng, N)
+    x = rng.standard_normal((T, K), dtype=np.float32)
+    y = out_buffer(T, N)
+    say("wide tiles, last row blocks", kind, T)
+    ops.launch_gemm_tiled_q(torch.from_numpy(x).cuda(), W.view, bd, T, K, N, y)
+    torch.cuda.synchronize()
+    check_sampled(y, x, W, T, rng, f"last row blocks fp32 kind={kind} T={T}", bb)
+    xb = O.f32_to_bf16(x)
+    y = out_buffer(T, N)
+    ops.launch_gemm_bf16x(torch.from_numpy(xb.view(np.int16)).cuda(), W.view, bd, T, K, N, y)
+    torch.cuda.synchronize()
+    check_sampled(y, O.bf16_to_f32(xb), W, T, rng, f"last row blocks bf16 kind={kind} T={T}", bb)
+
+
+# (bf16 at 8192 x 4096 runs the narrow tiles, at 18944 x 3584 128-row wide
+# ones, at 3587 x 18944 256-row ones, whose last tile has 4 of 8 row blocks)
+NON_FINITE = [(8192, 4096, 513), (18944, 3584, 450), (3587, 18944, 700)]
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("N,K,T", NON_FINITE)
+def test_wide_tiles_non_finite_rows(kind, N, K, T):
     """A row with inf or NaN gives a non-finite output row and leaves the
     other rows as they are."""
-    N, K, T = 8192, 4096, 513
     rng = np.random.default_rng(77 + kind)
     W = QFix(rng, N, K, kind, sd=0.02)
     x = rng.standard_normal((T, K), dtype=np.float32)
     bad = x.copy()
-    bad[5, 100], bad[300, K - 1], bad[512, 0] = np.inf, np.nan, -np.inf
-    rows = [5, 300, 512]
+    bad[5, 100], bad[300, K - 1], bad[T - 1, 0] = np.inf, np.nan, -np.inf
+    rows = [5, 300, T - 1]
     for bf16 in (False, True):
         ys = []
         for v in (x, bad):

@@ -15,11 +15,17 @@ from tests.gpu_util import QFix, bias_of, check_linear, out_buffer, say
 pytestmark = pytest.mark.gpu
 
 
-# (row counts of the matrices, K): K = 6144 / 8960 / 12800 take the kernel at
-# any row count (G >= 48), the others from 17 rows on or on enough tiles
+# (row counts of the matrices, K): the kernel serves MANY at every row count
+# of the test, LONG up to 16 rows, and of SOME only part (test_routes.py
+# asserts which; the other kernels the rest)
+MANY = [((16389, 1, 40), 1024), ((1025, 17), 16384), ((1030,), 16640)]
+LONG = [((1,), 16640), ((17,), 16384), ((250, 33), 16640)]
+SOME = [((1,), 6144), ((17,), 8960), ((250, 33), 8960), ((1025,), 6400), ((1024, 500), 256),
+        ((4609,), 3584), ((16400,), 512), ((1100, 16, 5), 12800)]
+
+
 @pytest.mark.parametrize("kind", [0, 1])
-@pytest.mark.parametrize("Ns,K", [((1,), 6144), ((17,), 8960), ((250, 33), 8960), ((1025,), 6400), ((1024, 500), 256),
-                                  ((4609,), 3584), ((16400,), 512), ((1100, 16, 5), 12800)])
+@pytest.mark.parametrize("Ns,K", SOME + MANY + LONG)
 def test_rows_edges(kind, Ns, K):
     rng = np.random.default_rng(sum(Ns) + K + kind)
     Ws = [QFix(rng, N, K, kind, sd=0.02) for N in Ns]
@@ -37,10 +43,12 @@ def test_rows_edges(kind, Ns, K):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [5, 16, 32])
-def test_rows_non_finite(kind, M):
+@pytest.mark.parametrize("K", [8960, 16384])
+def test_rows_non_finite(kind, M, K):
     """inf and NaN in a row make that row non-finite and leave the others
-    bit for bit as they are."""
-    N, K = 1600, 8960
+    bit for bit as they are (K = 8960 at 5 rows on the 1-row kernel, the
+    rest on this one)."""
+    N = 1600
     rng = np.random.default_rng(3 + kind)
     W = QFix(rng, N, K, kind, sd=0.02)
     x = rng.standard_normal((M, K), dtype=np.float32)
@@ -57,10 +65,15 @@ def test_rows_non_finite(kind, M):
     assert not torch.isfinite(ys[1][[1, M - 1]]).any()
 
 
-def test_rows_small_scratch():
+# (N of 3 ranges' sums inside and beyond the no-allocation scratch)
+SCRATCH = dict(inside=38000, beyond=48000, K=6144, M=32)
+
+
+@pytest.mark.parametrize("N", [SCRATCH["inside"], SCRATCH["beyond"]])
+def test_rows_small_scratch(N):
     """More range sums than the no-allocation scratch holds: another route,
     the same result."""
-    N, K, M, kind = 38000, 6144, 32, 1
+    K, M, kind = SCRATCH["K"], SCRATCH["M"], 1
     rng = np.random.default_rng(11)
     W = QFix(rng, N, K, kind, sd=0.02)
     x = rng.standard_normal((M, K), dtype=np.float32)
