@@ -13,19 +13,23 @@ Routes covered (dispatch in infer_amd/csrc/iq_gemm.hip / iq_gemv.hip):
     tiles >= 2 x CUs, i.e. the 128 x 128 tile instance (NJ = 2, BM = 128),
     and on 3584 x 18944 (config 5's down, K = 18944), bf16 and fp32
     activations, int8 and int4;
-  * gate|up (2 x 18944 x 3584) in one iq_gemv_multi call at 9, 12 and 16
-    rows (int4 on gemvq: 32-row tiles on the 32 x 32 matrix instruction,
+  * at 5..32 rows every call of an even number of 128-column groups below
+    takes gemvw (also those of the 7B layers), except narrow ones; the
+    kernels that serve the odd numbers are reached by the same calls one
+    group shorter or longer (K = 1152, 3456, 19072):
+  * gate|up (2 x 18944 rows) in one iq_gemv_multi call at 9, 12 and 16 rows
+    (odd: int4 on gemvq: 32-row tiles on the 32 x 32 matrix instruction,
     both terms of all 16 rows in one operand; int8 on gemvr) and at 1 row;
   * the int8 lm_head 152064 x 3584 at 1, 5 and 16 rows, and wide calls
-    (>= 4096 tiles) at 5..16 rows (gemvr at 5..6, gemvs at 7..16: operands
-    shared through LDS over 8 tiles), both kinds, with ragged row counts and
-    biases;
-  * 17..32 rows on gemvq's two 16-row blocks (7B gate|up and down, ragged
+    (>= 4096 tiles) at 5..16 rows (odd: gemvr at 5..6, gemvs at 7..16:
+    operands shared through LDS over 8 tiles, int4 gemvq), both kinds, with
+    ragged row counts and biases;
+  * 17..32 rows (odd: gemvq's two 16-row blocks; gate|up and down, ragged
     matrices, the fp32 GEMM entry);
-  * gate|up and down at 5..8 rows and down at 9..16 take gemvr (a K range
+  * gate|up and down at 5..8 rows and down at 9..16 (odd: gemvr, a K range
     requested at once, the f16 split operands made from x inside the
-    kernel), gate|up at 9..16 gemvq, with a non-finite activation in two
-    rows;
+    kernel), gate|up at 9..16 (odd: gemvq for int4), with a non-finite
+    activation in two rows, as also on gemvs and gemvh;
   * every other 7B decode matrix at 16 rows;
   * every row count where the routing changes, on narrow, wide and long-K
     shapes, and every T where the prefill GEMM's choices change, both
@@ -196,12 +200,13 @@ def test_one_row_short_tiles(kind):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [9, 16])
-def test_qkv_7b_multi_gemvh(kind, M):
+@pytest.mark.parametrize("K", [3584, 3456])
+def test_qkv_7b_multi_gemvh(kind, M, K):
     """q|k|v of one 7B layer (3584 + 512 + 512 rows x 3584, 288 tiles) in
-    one iq_gemv_multi call at 9..16 rows: the preparation launch and gemvh
-    on two tiles per workgroup, two groups in flight per wave."""
+    one iq_gemv_multi call at 9..16 rows, on gemvw; with 27 groups, the
+    preparation launch and gemvh on two tiles per workgroup, two groups in
+    flight per wave."""
     rng = np.random.default_rng(4600 + 20 * kind + M)
-    K = 3584
     Ws = [Packed(rng, n, K, kind) for n in (3584, 512, 512)]
     x = rng.standard_normal((M, K), dtype=np.float32)
     ys = [out_buffer(M, W.rows) for W in Ws]
@@ -228,13 +233,14 @@ def test_lm_head_int8(M):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [5, 7, 8, 9, 10, 11, 13, 16])
-def test_wide_call_5_to_16_rows(kind, M):
+@pytest.mark.parametrize("K", [1024, 1152])
+def test_wide_call_5_to_16_rows(kind, M, K):
     """Over 4096 16-row tiles (here 65541 rows, the last tile ragged, and a
-    second matrix in the same call) at 5..16 rows: the gemvr route on the
-    packed hi/lo operands (5..6 rows), the gemvs route on 16-row operand
-    blocks (int8 at 7..16) and gemvq straight from x (int4 at 7..16)."""
+    second matrix in the same call) at 5..16 rows: gemvw, and with nine
+    groups the gemvr route on the packed hi/lo operands (5..6 rows), the
+    gemvs route on 16-row operand blocks (int8 at 7..16) and gemvq straight
+    from x (int4 at 7..16)."""
     rng = np.random.default_rng(4096 + 10 * M + kind)
-    K = 1024
     Ws = [Packed(rng, 65541, K, kind), Packed(rng, 300, K, kind)]
     bias_bits = [O.seeded_bf16(rng, (W.rows,), 0.5) for W in Ws]
     bias = [torch.from_numpy(b.view(np.int16)).cuda() for b in bias_bits]
@@ -249,14 +255,14 @@ def test_wide_call_5_to_16_rows(kind, M):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [9, 16])
-def test_gemvq_ragged_matrices(kind, M):
-    """gemvq (int4; int8 takes gemvr) at 1024..4095 16-row tiles and 9..16
-    rows, on matrices whose rows are not a multiple of 32: 20005 + 309 + 48 rows in one call, with
+@pytest.mark.parametrize("K", [1024, 1152])
+def test_gemvq_ragged_matrices(kind, M, K):
+    """gemvw, and with nine groups gemvq (int4; int8 takes gemvr), at
+    1024..4095 16-row tiles and 9..16 rows, on matrices whose rows are not a multiple of 32: 20005 + 309 + 48 rows in one call, with
     biases, so the 32-row tiles of the second and third matrix start inside
     the first one's last 16-row tile pair and the split-K partials of each
     land in the 16-row tile order of the reduction."""
     rng = np.random.default_rng(3232 + 10 * M + kind)
-    K = 1024
     Ws = [Packed(rng, N, K, kind) for N in (20005, 309, 48)]
     bias_bits = [O.seeded_bf16(rng, (W.rows,), 0.5) for W in Ws]
     bias = [torch.from_numpy(b.view(np.int16)).cuda() for b in bias_bits]
@@ -271,13 +277,15 @@ def test_gemvq_ragged_matrices(kind, M):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [17, 24, 32])
-def test_gemvq_two_row_blocks(kind, M):
-    """17..32 rows on gemvq's two 16-row blocks: 7B gate|up (one call),
-    down (K = 18944) and q|k|v (a narrow call of three matrices) with
-    biases, ragged matrices (20005 + 309 + 48 rows, K = 1024) in one call,
-    and the fp32 GEMM entry (iq_gemm) on 7B gate."""
+@pytest.mark.parametrize("hidden,inner,short", [(3584, 18944, 1024), (3456, 19072, 1152)])
+def test_gemvq_two_row_blocks(kind, M, hidden, inner, short):
+    """17..32 rows on gemvw and, where the group counts are odd, on gemvq's
+    two 16-row blocks: 7B gate|up (one call), down (K = 18944) and q|k|v (a
+    narrow call of three matrices) with biases, ragged matrices (20005 + 309
+    + 48 rows, K = 1024) in one call, and the fp32 GEMM entry (iq_gemm) on
+    7B gate."""
     rng = np.random.default_rng(1732 + 10 * M + kind)
-    cases = ((3584, (18944, 18944)), (18944, (3584,)), (3584, (3584, 512, 512)), (1024, (20005, 309, 48)))
+    cases = ((hidden, (18944, 18944)), (inner, (3584,)), (hidden, (3584, 512, 512)), (short, (20005, 309, 48)))
     for K, Ns in cases:
         Ws = [Packed(rng, N, K, kind) for N in Ns]
         x = rng.standard_normal((M, K), dtype=np.float32)
@@ -289,7 +297,7 @@ def test_gemvq_two_row_blocks(kind, M):
         torch.cuda.synchronize()
         for i, (W, y) in enumerate(zip(Ws, ys)):
             check_sampled(y, x, W, M, rng, f"gemvq M={M} K={K} N={Ns[i]} kind={kind}", bias_bits[i])
-    K, N = 3584, 18944
+    K, N = hidden, 18944
     W = Packed(rng, N, K, kind)
     x = rng.standard_normal((M, K), dtype=np.float32)
     x[M - 1, 77] = np.inf
@@ -420,13 +428,15 @@ def test_random_shapes_across_routes(kind):
             check_sampled(y, x, W, M, rng, f"random {Ns[i]}x{K} M={M} kind={kind} [{i}]", bias_bits=bb)
 
 
-def test_gemvq_looped_k_ranges():
-    """gemvq where one K range per workgroup would need more partial sums
-    than the workspace holds, so each workgroup loops over several ranges:
-    the int8 lm_head at 32 rows (per-stream workspace) and int4 7B gate at
-    32 rows through iq_gemv_noalloc (the static array's smaller capacity)."""
+@pytest.mark.parametrize("K", [3584, 3456])
+def test_gemvq_looped_k_ranges(K):
+    """gemvq (27 groups; gemvw serves 28) where one K range per workgroup
+    would need more partial sums than the workspace holds, so each workgroup
+    loops over several ranges: the int8 lm_head at 32 rows (per-stream
+    workspace) and int4 7B gate at 32 rows through iq_gemv_noalloc (the
+    static array's smaller capacity)."""
     rng = np.random.default_rng(3232032)
-    M, K = 32, 3584
+    M = 32
     W = Packed(rng, 152064, K, 0)
     x = rng.standard_normal((M, K), dtype=np.float32)
     y = out_buffer(M, W.rows)
@@ -445,12 +455,12 @@ def test_gemvq_looped_k_ranges():
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [6, 12])
-def test_in_kernel_operands_unaligned_x(kind, M):
-    """gemvr (6 rows) and gemvq (12 rows), which read fp32 x themselves, on
-    an activation block that starts 4 bytes past a 16-byte boundary (7B
+@pytest.mark.parametrize("K", [3584, 3456])
+def test_in_kernel_operands_unaligned_x(kind, M, K):
+    """gemvw, and with 27 groups gemvr (6 rows; int8 also at 12) and gemvq
+    (int4 at 12), which read fp32 x themselves, on an activation block that starts 4 bytes past a 16-byte boundary (7B
     gate|up in one call)."""
     rng = np.random.default_rng(4444 + 10 * M + kind)
-    K = 3584
     Ws = [Packed(rng, 18944, K, kind) for _ in range(2)]
     x = rng.standard_normal((M, K), dtype=np.float32)
     buf = torch.zeros(M * K + 4, dtype=torch.float32, device="cuda")
@@ -467,12 +477,17 @@ def test_in_kernel_operands_unaligned_x(kind, M):
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("M", [6, 12])
-def test_gemvr_nonfinite_rows(kind, M):
-    """gemvr (7B gate|up and down shapes at 6 and 12 rows): an inf in row 0
-    and a NaN in row 1 make every output of those rows non-finite; the
-    other rows match the oracle."""
+@pytest.mark.parametrize("shapes", [((3584, (18944, 18944)), (18944, (3584,))),
+                                    ((3456, (18944, 18944)), (19072, (3584,))),
+                                    ((1152, (65541,)), (3456, (3584, 512, 512)))])
+def test_gemvr_nonfinite_rows(kind, M, shapes):
+    """7B gate|up and down shapes at 6 and 12 rows, on gemvw and with odd
+    group counts on gemvr (gemvq for int4 gate|up at 12), and at 12 rows a
+    wide call on gemvs (int4 gemvq) and q|k|v on gemvh: an inf in row 0 and a
+    NaN in row 1 make every output of those rows non-finite; the other rows
+    match the oracle."""
     rng = np.random.default_rng(7100 + 10 * M + kind)
-    for K, Ns in ((3584, (18944, 18944)), (18944, (3584,))):
+    for K, Ns in shapes:
         Ws = [Packed(rng, N, K, kind) for N in Ns]
         x = rng.standard_normal((M, K), dtype=np.float32)
         x[0, K - 3] = np.inf
