@@ -1,9 +1,10 @@
 """Chain stages at 5..32 rows on the kernel whose waves hold their
 activations (gemvw_kernel's chain instances): one wave a workgroup (more rows
-than its row factors' first set), two groups a wave, four, K split (down and,
-from 17 rows, 28 groups), both kinds, SwiGLU pairs, residuals, the sums of
-squares handed to the next stage; stage by stage against the oracle on the
-chain's own inputs."""
+than its row factors' first set), two groups a wave, four, K split (down of
+128 groups at any row count; from 17 rows also 36 and 28 groups), both kinds,
+SwiGLU pairs, residuals, the sums of squares handed to the next stage; stage
+by stage against the oracle on the chain's own inputs.  The narrow down
+stage of 36 groups at 5..16 rows runs gemvh."""
 import numpy as np
 import pytest
 import torch
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("B", [5, 8, 9, 17, 24, 32])
 @pytest.mark.parametrize("kind", [0, 1])
-@pytest.mark.parametrize("H,I,nh,nkv", [(256, 512, 2, 1), (1024, 2304, 8, 2), (1536, 3072, 12, 2), (3584, 4608, 28, 4)])
+@pytest.mark.parametrize("H,I,nh,nkv", [(256, 512, 2, 1), (1024, 2304, 8, 2), (1536, 3072, 12, 2), (3584, 4608, 28, 4),
+                                         (256, 16384, 2, 1)])
 def test_chain_rows_holding_waves(H, I, nh, nkv, kind, B):
     rng = np.random.default_rng(H + 7 * B + kind)
     host, dev = make_model(rng, H=H, I=I, nh=nh, nkv=nkv, hd=128, V=1000, L=2, kind=kind, head_kind=0)
