@@ -785,8 +785,8 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
             continue;
         }
         if (rows > 1) {
-            // B rows: the rows GEMV (gemvr / gemvq with the input transform)
-            // and epi_kernel
+            // B rows: the rows GEMV with the input transform (rows_setup) and
+            // epi_kernel, or one of the routes below
             for (int i = 0; i < a.n; i++) {
                 const iq_view& Wi = a.W[i];
                 hs.W[i] = QView{Wi.kind, Wi.rows, Wi.cols, Wi.groups, Wi.q, Wi.scales,

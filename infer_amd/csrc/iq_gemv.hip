@@ -703,7 +703,6 @@ __global__ __launch_bounds__(512) void gemvb_kernel(const GemvParams p) {
     const uint16_t* srow = p.scales + rc * G;
     const uint8_t* zrow = KIND == 1 ? p.zeros + rc * G : nullptr;
     const int xrec = M * kLimbRec;                 // bytes of limbs per group (all rows)
-    const int xch = GC * xrec / 16;                // 16-byte chunks per activation chunk
     int4* msb = reinterpret_cast<int4*>(xsb + GC * xrec);
     constexpr int XPT = (GC * kMaxRowsGemv * kLimbRec / 16 + NT - 1) / NT;  // max chunks per thread
     if (tid < 4) reinterpret_cast<uint32_t*>(xzero)[tid] = 0u;
@@ -1343,7 +1342,6 @@ hipError_t launch_gemv1(const float* x, const QView* W, const uint16_t* const* b
     // the K ranges' sums, in range order, + bias
     GemvParams pr = p;
     pr.S = pl.kr;
-    const int64_t cnt = int64_t(M) * tiles * 16;
     launch_gemvt_reduce(pr, stream);
     return hipGetLastError();
 }
@@ -1496,10 +1494,7 @@ bool launch_gemvt(const QView* W, const uint16_t* const* bias, float* const* y, 
         p.ntiles = tiles;
         if (W[0].kind == 1) launch_gemvt_k<1>(p, pl, stream);
         else launch_gemvt_k<0>(p, pl, stream);
-        if (pl.ks > 1) {
-            const int64_t cnt = int64_t(mb) * tiles * 16;
-            launch_gemvt_reduce(p, stream);
-        }
+        if (pl.ks > 1) launch_gemvt_reduce(p, stream);
         *err = hipGetLastError();
         if (*err != hipSuccess) return true;
     }
@@ -1522,14 +1517,14 @@ bool launch_gemvt(const QView* W, const uint16_t* const* bias, float* const* y, 
 // i = l % 16, q = l / 16) holding x[16 b + i][128 g + 32 q + 8 j + c(e)] for
 // its 8 slots e, c(e) = perm8(e) for int4 weights (the order in which
 // dq_int4_x8 leaves the nibbles) and e for int8; and per (b, g) the 16
-// factors 2^-k (NaN when the group holds a non-finite value, so the outputs
-// it reaches are NaN).  Every A operand is then one contiguous 1 KiB load.
+// factors 2^-k (a non-finite value is non-finite in its operands, and so are
+// its row's outputs).  Every A operand is then one contiguous 1 KiB load.
 constexpr int kHGroupBytes = 4 * 2 * 64 * 16;  // prepared bytes per (block, group)
 
 // The f16 split of one lane's 8 values of a (row, group): all 16 lanes of a
 // DPP row hold the group's 128 values (the group maximum is taken across
 // them).  ho / lo: the hi and lo terms in operand slot order (perm8 for int4
-// weights); fac: 2^-k, or NaN when the group holds a non-finite value.
+// weights); fac: 2^-k.
 template <bool PERM>
 __device__ __forceinline__ void xh_split8(const float (&v)[8], half8_t& ho, half8_t& lo, float& fac) {
     // largest |x| over the 16 lanes (max ignores a NaN; an infinity stays)
@@ -2502,7 +2497,8 @@ __global__ __launch_bounds__(512, 2) void gemvw_kernel(const GemvParams p) {
         }
     };
     // (the instance whose registers the operands, the prologue and int8
-    // weights would overfill requests its second tile after the conversion)
+    // weights overfill requests its second tile after the conversion; 13 of
+    // its 256 registers still spill, to 56 bytes of scratch a lane)
     constexpr bool TIGHT = PRO && KIND == 0 && MB2 == 2 && NG == 4;
     constexpr int EARLY = TIGHT ? 1 : S::D;
 #pragma unroll
@@ -2792,7 +2788,6 @@ bool launch_gemvr(const float* x, const QView* W, const uint16_t* const* bias, f
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
-        const int64_t outs = int64_t(M) * tiles * 16;
         launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
@@ -2863,7 +2858,6 @@ bool launch_gemvq(const float* x, const QView* W, const uint16_t* const* bias, f
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
-        const int64_t outs = int64_t(M) * tiles * 16;
         launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
@@ -2905,7 +2899,6 @@ bool launch_gemvs(const QView* W, const uint16_t* const* bias, float* const* y, 
     else gemvs_kernel<0><<<grid, 512, 0, stream>>>(p);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && S > 1) {
-        const int64_t outs = int64_t(M) * tiles * 16;
         launch_gemvt_reduce(p, stream);
         e = hipGetLastError();
     }
@@ -3251,9 +3244,9 @@ hipError_t launch_gemv(const float* x, const QView& W, const uint16_t* bias, int
 // ------------------------------------------------------------------ B-row chain stages
 namespace {
 
-// The kernel and K ranges of a B-row chain stage (the rows GEMV of
-// launch_gemv_multi: gemvr, or gemvq from 17 rows and for wide int4 calls
-// from 9), every range's sums written to part [S][M][tiles * 16].
+// The kernel and K ranges of a B-row chain stage (gemvw from 5 rows on; where
+// its sums do not fit, and at 2..4 rows, gemvr, or gemvq from 17 rows and for
+// wide int4 calls from 9), every range's sums written to part [S][M][tiles * 16].
 struct RowsSetup {
     GemvParams p{};
     bool q = false;  // gemvq (else gemvr)

@@ -110,10 +110,11 @@ inline GwPlan gemvw_plan(int64_t G, int M, int units, int cus) {
 // 11.4; 1024 x 7168 16.9 -> 12.6); 9..16 rows on long rows (1.5B down, G =
 // 70, int8 20.9 -> 11.0, int4 15.2 -> 10.2) or where tiles x groups fill the
 // card (7B q|k|v, 288 x 28, 12.3 -> 11.4; o, 224 x 28, int4 9.7 kept against
-// 10.4, int8 11.9 -> 11.1; 7168 x 1024, 448 x 8, 7.6 kept against 8.9); 5..8
-// rows wherever the 1-row kernel's exact integer sums do not serve (on those
-// narrow calls, where gemvw would be up to 25 % faster at 8 rows, its error
-// is 1.2 to 1.4 times theirs).
+// 10.4, int8 11.9 -> 11.1; 7168 x 1024, 448 x 8, 7.6 kept against 8.9: the
+// two lines lie closely about o's 6272, between the two other shapes, and
+// nothing nearer was measured); 5..8 rows wherever the 1-row kernel's exact
+// integer sums do not serve (on those narrow calls, where gemvw would be up
+// to 25 % faster at 8 rows, its error is 1.2 to 1.4 times theirs).
 inline bool gemvw_preferred(int M, int tiles, int64_t K, int kind, int cus) {
     const int64_t G = K / 128;
     if (M < 5 || M > kMaxRowsGemv || K % 128 || G % 2) return false;
@@ -131,9 +132,11 @@ inline bool gemvw_preferred(int M, int tiles, int64_t K, int kind, int cus) {
 // to take (> 1: every tile is split).  us: the estimate; above 1e29 when no
 // plan fits.  The times per group and round are measured: bf16 at bm = 256 /
 // 128, 16384 x 4096 at T = 1024 143 / 195 us, fp32 246 us (one, two and two
-// rounds of 32 groups); the sums cost 8 bytes a float at 9 TB/s (they stay
-// in the last-level cache) and a launch.  Splitting only the last, partly
-// filled round: 7B gate at T = 1024, bf16 222 -> 171 us, fp32 307 -> 296.
+// rounds of 32 groups; int8 codes, and int4 takes up to a quarter longer in
+// bf16, 7B gate's product 160 / 199 us, which the estimate leaves out); the
+// sums cost 8 bytes a float at 9 TB/s (they stay in the last-level cache) and
+// a launch.  Splitting only the last, partly filled round: 7B gate at T =
+// 1024, bf16 222 -> 171 us, fp32 307 -> 296.
 struct GemmwPlan {
     int bm = 0, tiles_m = 0, tiles_n = 0, full = 0, splits = 1, gch = 0;
     double us = 1e30;
