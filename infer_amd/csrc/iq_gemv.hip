@@ -1057,10 +1057,14 @@ __global__ __launch_bounds__(512) void gemvt_kernel(const GemvParams p) {
 // latency of a launch and of ceil(S / 8) loads; the arithmetic around them
 // (a column and a 64-bit division per thread) cost too: with this form and
 // the preparation's grid over (row, groups) instead of divisions, 8 layers
-// of 7B int4 at 16 rows 638 -> 628 us.
-__global__ __launch_bounds__(128) void gemvt_reduce_kernel(const GemvParams p) {
+// of 7B int4 at 16 rows 638 -> 628 us.  A workgroup takes 256 columns, as the
+// kernels that write the sums do: the two then tend to run on the same XCD,
+// whose L2 holds them (whole calls with 512 / 256 columns: 4096 x 1152 int4
+// at 24 / 32 rows 10.1 / 11.5 -> 9.0 / 9.4 us, 6144 x 2176 int8 at 32 rows
+// 20.3 -> 15.7, 5000 x 1920 int4 at 17 / 24 rows 13.6 / 14.7 -> 12.6 / 13.4).
+__global__ __launch_bounds__(64) void gemvt_reduce_kernel(const GemvParams p) {
     const int ld = p.ntiles * 16, m = blockIdx.y;
-    const int c = (int(blockIdx.x) * 128 + int(threadIdx.x)) * 4;
+    const int c = (int(blockIdx.x) * 64 + int(threadIdx.x)) * 4;
     if (c >= ld) return;
     const TileSel ts = select_tile(p, c >> 4);
     const int64_t row = ts.row0 + (c & 15);
@@ -1079,7 +1083,7 @@ __global__ __launch_bounds__(128) void gemvt_reduce_kernel(const GemvParams p) {
 }
 
 void launch_gemvt_reduce(const GemvParams& p, hipStream_t stream) {
-    gemvt_reduce_kernel<<<dim3(unsigned((p.ntiles * 4 + 127) / 128), unsigned(p.M)), 128, 0, stream>>>(p);
+    gemvt_reduce_kernel<<<dim3(unsigned((p.ntiles * 4 + 63) / 64), unsigned(p.M)), 64, 0, stream>>>(p);
 }
 
 // y[m, n] = sum over slices s of part[s, m, n] (in slice order) + bias[n].
