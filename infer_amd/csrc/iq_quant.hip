@@ -161,13 +161,23 @@ __device__ __forceinline__ uint32_t pack4_b0(int c0, int c1, int c2, int c3) {
 // byte at a time.  Bound by HBM like the whole-group form (element by
 // element loads and byte stores in all lanes: 15872 x 2146 int4 52.5 ->
 // 28.0 us, 15872 x 2147 int8 56.5 -> 26.9).
-template <int KIND, bool RAGGED>
+// SHARED: ragged rows of up to 4 groups, 8, 4 or 2 of them an item (`sh`: the
+// log2 of the group slots that a row takes of the item's 8).  With one row an
+// item half of the lanes or more idled, and inputs in the last-level cache
+// took longer than with the element loads (per row / shared: 200000 x 100
+// int4 104 -> 20 us, 40000 x 200 int8 23.3 -> 10.7, 263000 x 258 int8 120 ->
+// 68, 150000 x 400 int4 80 -> 44; element loads 95, 20.7, 116 and 78).
+template <int KIND, bool RAGGED, bool SHARED>
 __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __restrict__ w, int64_t rows,
-                                                              int64_t cols, int64_t G, int64_t octs,
+                                                              int64_t cols, int64_t G, int64_t octs, int sh,
                                                               uint8_t* __restrict__ q, uint16_t* __restrict__ scales,
                                                               uint8_t* __restrict__ zeros) {
     const int lane = threadIdx.x & 63, sub = lane & 7;
-    const int64_t items = rows * octs;
+    // this lane's group of an item, and (SHARED) its row
+    const int gl = SHARED ? (lane >> 3) & ((1 << sh) - 1) : lane >> 3, rl = SHARED ? lane >> (3 + sh) : 0;
+    const int per = SHARED ? 8 >> sh : 1;  // rows of an item
+    const int64_t blocks = SHARED ? (rows + per - 1) / per : rows;
+    const int64_t items = blocks * octs;
     const int64_t stride = int64_t(gridDim.x) * (kQThreads / 64);
     const int64_t first0 = int64_t(blockIdx.x) * (kQThreads / 64) + (threadIdx.x >> 6);
     const int64_t first = (int64_t(__builtin_amdgcn_readfirstlane(uint32_t(first0 >> 32))) << 32) |
@@ -175,7 +185,7 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
     if (first >= items) return;
     const int64_t sr = stride / octs, so = stride % octs;
     struct Cursor {
-        int64_t r, o;
+        int64_t r, o;  // row block, 8 groups of it
     };
     auto advance = [&](Cursor& c) {
         c.r += sr;
@@ -189,15 +199,19 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
         uint4 a, b;
     };
     auto fetch = [&](const Cursor& c) {
-        const bool rok = c.r < rows;
+        const bool rok = c.r < blocks;
         // RAGGED: a resource over the item's columns, whose last chunk runs
-        // into the next row; lane l's 16 columns at 32 l
-        const int64_t r = rok ? c.r : 0, col0 = c.o * (8 * kGroup);
-        const int64_t avail = RAGGED ? std::min<int64_t>(rows * cols - r * cols - col0, 8 * kGroup + 16) : cols;
+        // into the next row
+        const int64_t r = rok ? c.r * per : 0, col0 = c.o * (8 * kGroup);
+        const int64_t span = SHARED ? per * cols + 16 : 8 * kGroup + 16;
+        const int64_t avail = RAGGED ? std::min<int64_t>((rows - r) * cols - col0, span) : cols;
         const rsrc_t rw = make_rsrc(w + r * cols + (RAGGED ? col0 : 0), rok ? avail * 2 : 0);
-        const int64_t g = c.o * 8 + (lane >> 3);
+        const int64_t g = c.o * 8 + gl;
         uint32_t off;
-        if (RAGGED) off = col0 + lane * 16 < cols ? uint32_t(lane * 32) : kOob;
+        if (SHARED)
+            off = r + rl < rows && gl * kGroup + sub * 16 < int(cols) ? uint32_t(rl * int(cols) + gl * kGroup + sub * 16) * 2
+                                                                      : kOob;
+        else if (RAGGED) off = col0 + lane * 16 < cols ? uint32_t(lane * 32) : kOob;
         else off = g < G ? uint32_t((g * kGroup + sub * 16) * 2) : kOob;
         Raw x;
         x.a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
@@ -208,20 +222,20 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
         return x;
     };
     auto process = [&](const Cursor& cc, const Raw& cur) {
-        const int64_t r = cc.r;
-        const int64_t g = cc.o * 8 + (lane >> 3);
-        const bool gvalid = g < G;
+        const int64_t r = SHARED ? cc.r * per + rl : cc.r;
+        const int64_t g = cc.o * 8 + gl;
+        const bool gvalid = g < G && (!SHARED || r < rows);
         uint32_t wd[8] = {cur.a.x, cur.a.y, cur.a.z, cur.a.w, cur.b.x, cur.b.y, cur.b.z, cur.b.w};
         const int64_t c0 = g * kGroup + sub * 16;
         const int64_t left = cols - c0;  // columns of the row from this lane's first on
         const bool edge = RAGGED && (cc.o + 1) * 8 * kGroup > cols;  // wave-uniform: the row ends here
         if (edge) {
-            if (r + 1 == rows && (cols & 1)) {
+            if ((cols & 1) && (cc.r + 1) * per >= rows) {
                 // the matrix ends inside a 4-byte word, which the buffer
                 // resource cuts off whole: its last value on its own
-                const uint32_t e = w[r * cols + cols - 1];
+                const uint32_t e = w[rows * cols - 1];
 #pragma unroll
-                for (int i = 0; i < 8; i++) wd[i] = left == 2 * i + 1 ? e : wd[i];
+                for (int i = 0; i < 8; i++) wd[i] = r + 1 == rows && left == 2 * i + 1 ? e : wd[i];
             }
 #pragma unroll
             for (int i = 0; i < 8; i++) wd[i] = left >= 2 * i + 2 ? wd[i] : (left == 2 * i + 1 ? wd[i] & 0xFFFFu : 0u);
@@ -361,15 +375,15 @@ __global__ __launch_bounds__(kQThreads) void quantize8_kernel(const uint16_t* __
         process(c0, ra);
         Cursor n = c2;
         advance(n);  // c0 + 3 strides
-        if (c1.r >= rows) break;
+        if (c1.r >= blocks) break;
         ra = fetch(n);
         process(c1, rb);
-        if (c2.r >= rows) break;
+        if (c2.r >= blocks) break;
         Cursor n1 = n;
         advance(n1);
         rb = fetch(n1);
         process(c2, rc);
-        if (n.r >= rows) break;
+        if (n.r >= blocks) break;
         c0 = n;
         c1 = n1;
         c2 = n1;
@@ -414,14 +428,16 @@ hipError_t launch_quantize(const uint16_t* w, int64_t rows, int64_t cols, int ki
     // enough resident waves to stream; each walks items in strides of the grid
     const int64_t cap = int64_t(device_cu_count()) * 8;
     const int64_t octs = (G + 7) / 8;
-    const unsigned grid = unsigned(std::min<int64_t>((rows * octs + 3) / 4, cap));
-    if (cols % kGroup == 0) {
-        if (kind == 0) quantize8_kernel<0, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-        else quantize8_kernel<1, false><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-    } else {
-        if (kind == 0) quantize8_kernel<0, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-        else quantize8_kernel<1, true><<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, q, scales, zeros);
-    }
+    // ragged rows of up to 4 groups share items (from 5 on more than half of
+    // an item's lanes have work: 100000 x 514 int8 51 us, element loads 109)
+    const bool ragged = cols % kGroup != 0, shared = ragged && G <= 4;
+    const int sh = !shared ? 3 : (G > 2 ? 2 : int(G) - 1);
+    const int64_t items = (rows + (8 >> sh) - 1) / (8 >> sh) * octs;
+    const unsigned grid = unsigned(std::min<int64_t>((items + 3) / 4, cap));
+    auto launch = [&](auto kernel) { kernel<<<grid, kQThreads, 0, stream>>>(w, rows, cols, G, octs, sh, q, scales, zeros); };
+    if (shared) kind == 0 ? launch(quantize8_kernel<0, true, true>) : launch(quantize8_kernel<1, true, true>);
+    else if (ragged) kind == 0 ? launch(quantize8_kernel<0, true, false>) : launch(quantize8_kernel<1, true, false>);
+    else kind == 0 ? launch(quantize8_kernel<0, false, false>) : launch(quantize8_kernel<1, false, false>);
     return hipGetLastError();
 }
 

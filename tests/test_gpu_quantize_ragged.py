@@ -1,6 +1,7 @@
 """On-device quantize of rows that are not whole 128-column groups, bit for
 bit against the oracle: rows ending inside a 16-column chunk, inside a 4-byte
-word and on either, the matrix's last value included; what follows a row
+word and on either, the matrix's last value included; rows short enough to
+share a wave; what follows a row
 (the next row, here with NaN and infinities in it) must not reach its codes;
 inputs off 16-byte alignment; nothing is written past the codes."""
 import numpy as np
@@ -16,7 +17,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 2), (2, 15), (5, 16), (3, 17), (9, 127), (4, 129), (7, 143), (6, 1023),
-                                       (5, 1024 + 16), (4, 1025), (3, 2049), (700, 300), (3000, 131)])
+                                       (5, 1024 + 16), (4, 1025), (3, 2049), (700, 300), (3000, 131),
+                                       # rows that share a wave: 8, 4 or 2, and a last wave with fewer
+                                       (8, 100), (17, 99), (9, 255), (4, 250), (5, 257), (2, 383), (3, 385), (2051, 511), (4, 513)])
 def test_quantize_ragged_rows(kind, rows, cols):
     if kind == 1:
         cols += cols % 2
