@@ -162,9 +162,9 @@ __global__ __launch_bounds__(BM == 256 ? 2 * kThreads : kThreads, BM == 256 ? 1 
     const int64_t nrows = p.N - n0 < BN ? p.N - n0 : BN;
     // kUnaligned: a row's last chunk runs into the next row's bytes, up to
     // the end of the whole matrix
-    const int64_t over = MODE == kUnaligned ? 16 : 0;
-    const int64_t xbytes = std::min(xrows * p.K * XE + over, (p.T - m0) * p.K * XE);
-    const int64_t wbytes = std::min(nrows * row_bytes + over, (p.N - n0) * row_bytes);
+    const int64_t xown = xrows * p.K * XE, wown = nrows * row_bytes;
+    const int64_t xbytes = MODE == kUnaligned ? std::min(xown + 16, (p.T - m0) * p.K * XE) : xown;
+    const int64_t wbytes = MODE == kUnaligned ? std::min(wown + 16, (p.N - n0) * row_bytes) : wown;
     const bool wlast = MODE == kUnaligned && n0 + BN >= p.N, xlast = MODE == kUnaligned && m0 + BM >= p.T;
     const rsrc_t rx = make_rsrc(XF32 ? static_cast<const void*>(p.xf + m0 * p.K)
                                      : static_cast<const void*>(p.xb + m0 * p.K), xbytes);
