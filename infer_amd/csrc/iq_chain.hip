@@ -122,7 +122,6 @@ struct HostStage {
     int rows = 1;
     int fused_r = 1;  // > 1: one stage_kernel launch of the R-row instance (rows <= R)
     bool wroute = false;  // B rows on rows of few groups: one gemvw launch (no epilogue launch)
-    bool hroute = false;  // B rows on a narrow stage: operand preparation + gemvh (no epilogue launch)
     QView W[kMaxStageMats];
     RowsIn in{};
     CEpi epi{};
@@ -671,9 +670,6 @@ struct Chain {
     float* rpart = nullptr;
     int64_t rpart_floats = 0;
     float* rssq = nullptr;
-    // narrow B-row stages: their prepared f16 operands (one stage at a time)
-    int8_t* hxq = nullptr;
-    float* hxmeta = nullptr;
 };
 
 int chain_create(const iq_stage* stages, int n, Chain** out) {
@@ -816,12 +812,12 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
             // groups, 17..32 rows up to 16): one launch with the epilogue in
             // it (1.5B int4 / int8 chains at 16 sequences 445 / 382 -> 386 /
             // 288 us, 7B int8 463 -> 362, with its down stage on gemvw's range
-            // sums).  Other narrow stages at 5..16 rows (an odd number of
-            // groups): the input transform into prepared f16 operands, then
-            // gemvh with bias, residual and per-tile sums of squares in its
-            // own epilogue
+            // sums).  Longer rows take the range sums and epi_kernel, narrow
+            // stages too (1.5B down, 70 groups, two layers and the head: int4
+            // at 5 / 16 sequences 155 / 172 -> 141 / 160 us against prepared
+            // operands and gemvh with the epilogue in it, int8 164 / 178 ->
+            // 146 / 165)
             hs.wroute = (a.out_op != IQ_OUT_RESIDUAL || a.n == 1) && chain_w_applies(hs.W, a.n, rows, pair);
-            hs.hroute = !hs.wroute && !pair && (a.out_op != IQ_OUT_RESIDUAL || a.n == 1) && chain_h_applies(hs.W, a.n, rows);
             continue;
         }
         // slices of whole 4-group blocks (measured: fewer, fatter waves beat
@@ -907,7 +903,7 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
         std::vector<int> producer(static_cast<size_t>(n), -1);
         auto ssq_count = [&](int e) {
             const HostStage& hp = prog[size_t(e)];
-            return (hp.fused_r > 1 || hp.hroute || hp.wroute) ? int((hp.st.mat[0].N + 15) / 16) : int((hp.epi.ncols + 255) / 256);
+            return (hp.fused_r > 1 || hp.wroute) ? int((hp.st.mat[0].N + 15) / 16) : int((hp.epi.ncols + 255) / 256);
         };
         for (const auto& l : links)
             if (rows_of(l.second) > 1 && ssq_count(l.first) <= 256) producer[size_t(l.second)] = l.first;
@@ -960,19 +956,6 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
             if (e != hipSuccess) return fail(e);
             ch->rpart_floats = part;
         }
-        size_t hxq = 0, hmeta = 0;
-        for (const HostStage& h : prog) {
-            if (!h.hroute) continue;
-            size_t xb = 0, mf = 0;
-            chain_h_bytes(h.W[0].groups, h.rows, &xb, &mf);
-            hxq = std::max(hxq, xb);
-            hmeta = std::max(hmeta, mf);
-        }
-        if (hxq) {
-            hipError_t e = hipMalloc(reinterpret_cast<void**>(&ch->hxq), hxq);
-            if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&ch->hxmeta), hmeta * sizeof(float));
-            if (e != hipSuccess) return fail(e);
-        }
     }
     ch->stages = std::move(prog);
     *out = ch;
@@ -982,17 +965,13 @@ int chain_create(const iq_stage* stages, int n, Chain** out) {
 hipError_t chain_run(const Chain* ch, hipStream_t stream) {
     for (const HostStage& h : ch->stages) {
         hipError_t e;
-        if (h.rows > 1 && h.fused_r == 1 && (h.hroute || h.wroute)) {
+        if (h.rows > 1 && h.fused_r == 1 && h.wroute) {
             if (h.own_ssq) {
                 const int K = int(h.W[0].cols);
                 ssq_kernel<<<dim3(unsigned(h.in.ssq_n), unsigned(h.rows)), 256, 0, stream>>>(h.in.x, K, h.in.ssq_n, h.ssq);
             }
-            if (h.wroute)
-                e = launch_chain_w(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.swiglu != 0, h.epi.res,
-                                   h.epi.ssq_out, stream);
-            else
-                e = launch_chain_h(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.res, h.epi.ssq_out, ch->hxq,
-                                   ch->hxmeta, stream);
+            e = launch_chain_w(h.W, h.st.nmat, h.rows, h.in, h.epi.bias, h.epi.y, h.epi.swiglu != 0, h.epi.res,
+                               h.epi.ssq_out, stream);
         } else if (h.rows > 1 && h.fused_r == 1) {
             e = run_rows_stage(h, ch->rpart, ch->rpart_floats, stream);
         } else {
@@ -1013,8 +992,6 @@ void chain_destroy(Chain* ch) {
     if (ch->partials) (void)hipFree(ch->partials);
     if (ch->rpart) (void)hipFree(ch->rpart);
     if (ch->rssq) (void)hipFree(ch->rssq);
-    if (ch->hxq) (void)hipFree(ch->hxq);
-    if (ch->hxmeta) (void)hipFree(ch->hxmeta);
     delete ch;
 }
 

@@ -1,10 +1,9 @@
 """Chain stages at 5..32 rows on the kernel whose waves hold their
 activations (gemvw_kernel's chain instances): one wave a workgroup (more rows
 than its row factors' first set), two groups a wave, four, K split (down of
-128 groups at any row count; from 17 rows also 36 and 28 groups), both kinds,
+36 and 128 groups at any row count, from 17 rows also 28 groups), both kinds,
 SwiGLU pairs, residuals, the sums of squares handed to the next stage; stage
-by stage against the oracle on the chain's own inputs.  The narrow down
-stage of 36 groups at 5..16 rows runs gemvh."""
+by stage against the oracle on the chain's own inputs."""
 import numpy as np
 import pytest
 import torch
