@@ -3006,7 +3006,10 @@ hipError_t launch_gemv_prepped(const QView& W, const uint16_t* bias, int M, floa
 hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* const* bias, float* const* y,
                              int n, int M, Workspace* ws, hipStream_t stream) {
     const int64_t K = W[0].cols, G = W[0].groups;
-    if (gemvw_preferred(M, total_tiles(W, n), K, W[0].kind, device_cu_count())) {
+    // (what asks for it needs it from 5 rows on only; eager 1-row calls are
+    // bound by the host)
+    const int cus = M > 4 ? device_cu_count() : 0;
+    if (gemvw_preferred(M, total_tiles(W, n), K, W[0].kind, cus)) {
         hipError_t e = hipSuccess;
         if (launch_gemvw(x, W, bias, y, n, M, ws, stream, &e)) {
             // gemvw leaves a preparation's buffers alone, but callers may
@@ -3088,7 +3091,7 @@ hipError_t launch_gemv_multi(const float* x, const QView* W, const uint16_t* con
         if (e != hipSuccess) return e;
         return launch_gemvh(W, bias, y, n, M, ws, stream);
     }
-    if (gemv1_rows_preferred(M, total_tiles(W, n), G, device_cu_count())) {
+    if (gemv1_rows_preferred(M, total_tiles(W, n), G, cus)) {
         // the 1-row kernel converts x itself; 2..8 rows share each weight
         // operand (no preparation launch, and the workspace's preparation
         // stays as it was)
