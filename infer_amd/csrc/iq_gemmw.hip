@@ -24,20 +24,21 @@
 //    while the previous group is multiplied (in a burst at the group's start
 //    they held up every wave's products: 1024 x 16384 x 4096 bf16 x int8
 //    170 -> 144 us), in an order of chunks that spreads a read's
-//    lanes over the banks (conflicts 4 % of the busy cycles).
+//    lanes over the banks (conflicts 3-7 % of the busy cycles).
 // The next group's codes are converted behind the last 16-row block of a
 // group, each operand where it has been used for the last time, so one set
 // of registers and one LDS buffer of codes suffice: 250 of 256 registers and
 // 160 KiB of LDS at 256 x 256 x int8.
 //
-// Measured (one MI355X, T = 1024, the narrow tiles -> these): bf16
-// activations, 7B gate 18944 x 3584 int8 / int4 213 / 216 -> 165 / 175 us
-// (842 / 795 TFLOP/s), down 3584 x 18944 261 / 270 -> 168 / 183; fp32
-// activations with their preparation, gate 381 / 357 -> 285 / 288 us, down
-// 393 / 372 -> 321 / 323.  1024 x 16384 x 4096, which fills one round of
-// tiles: 958 TFLOP/s of bf16 products, 1030 of fp16 ones; a dense bf16
-// library product of that size reaches about 1000, and zero activations run
-// 13 % faster than random ones, so power is part of what bounds it.
+// Measured (one MI355X, T = 1024, eight calls in a graph on one set of
+// weights, the narrow tiles -> these): bf16 activations, 7B gate 18944 x 3584
+// int8 / int4 190 / 203 -> 156 / 168 us (892 / 828 TFLOP/s), down 3584 x
+// 18944 241 / 260 -> 157 / 175; fp32 activations with their preparation,
+// gate 362 / 344 -> 281 / 282 us, down 350 / 355 -> 299 / 305.  1024 x 16384
+// x 4096, which fills one round of tiles: 958 TFLOP/s of bf16 products, 1030
+// of fp16 ones; a dense bf16 library product of that size reaches about
+// 1000, and zero activations run 13 % faster than random ones, so power is
+// part of what bounds it.
 #include <algorithm>
 
 #include "iq_gemm.h"
